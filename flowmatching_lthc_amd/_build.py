@@ -11,10 +11,11 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
-SOURCES = [os.path.join(PKG, "csrc", "lthc_kernels.hip")]
+SOURCES = [os.path.join(PKG, "csrc", n) for n in ("lthc_kernels.hip", "branch.hip")]
 LIB_DIR = os.path.join(PKG, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "liblthc_hip.so")
 ARCH = "gfx950"
@@ -25,7 +26,6 @@ HIPCC_FLAGS = [
     "-std=c++17",
     f"--offload-arch={ARCH}",
     "-fPIC",
-    "-shared",
     "-Xclang",
     "-target-feature",
     "-Xclang",
@@ -43,15 +43,23 @@ def hipcc() -> str:
 
 
 def build(verbose: bool = False) -> str:
-    """Compile every HIP source into LIB_PATH; returns the path."""
+    """Compile every HIP source (side by side) and link them into LIB_PATH; returns the path."""
     os.makedirs(LIB_DIR, exist_ok=True)
     tmp = LIB_PATH + ".tmp"
-    cmd = [hipcc(), *HIPCC_FLAGS, "-o", tmp, *SOURCES]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{' '.join(cmd)}\n{proc.stderr[-4000:]}")
-    if verbose and proc.stderr.strip():
-        print(proc.stderr, file=sys.stderr)
+    with tempfile.TemporaryDirectory(dir=LIB_DIR) as work:
+        objects = [os.path.join(work, os.path.basename(src) + ".o") for src in SOURCES]
+        cmds = [[hipcc(), *HIPCC_FLAGS, "-c", "-o", obj, src] for src, obj in zip(SOURCES, objects)]
+        procs = [subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True) for cmd in cmds]
+        outputs = [p.communicate()[0] for p in procs]
+        link = [hipcc(), f"--offload-arch={ARCH}", "-fPIC", "-shared", "-o", tmp, *objects]
+        for cmd, p, text in zip(cmds, procs, outputs):
+            if p.returncode != 0:
+                raise RuntimeError(f"hipcc failed ({p.returncode}):\n{' '.join(cmd)}\n{text[-4000:]}")
+            if verbose and text.strip():
+                print(text, file=sys.stderr)
+        proc = subprocess.run(link, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{' '.join(link)}\n{proc.stderr[-4000:]}")
     os.replace(tmp, LIB_PATH)
     return LIB_PATH
 

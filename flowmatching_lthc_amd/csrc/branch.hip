@@ -1,0 +1,11 @@
+// MI355X (gfx950) kernels and C ABI of the workspace transformer branch around the LTHC interface: RMSNorm +
+// modulate with its gated forms, the q/k norm + RoPE, the attention and the SwiGLU gate.  Declarations are in
+// include/lthc.h; the interface itself is lthc_kernels.hip.
+
+#include "common.inc"
+
+// RMSNorm + modulate (the decoder's input and the branch's pre-norms) with its gated forms.
+#include "norm_modulate.inc"
+#include "branch_ops.inc"
+// Fused q/k RMSNorm + RoPE and attention of the branch (matrix cores).
+#include "attention.inc"

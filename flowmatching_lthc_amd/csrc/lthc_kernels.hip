@@ -19,235 +19,9 @@
 // masked by a select), so a wavefront keeps all of a cell's loads in flight
 // instead of waiting on each one.
 
-#include <hip/hip_runtime.h>
-
-#include <stdint.h>
-
-#include <algorithm>
-#include <initializer_list>
-#include <numeric>
-#include <string>
-#include <type_traits>
-#include <utility>
-
-#include "../../include/lthc.h"
-
-#define LTHC_DEV __device__ __forceinline__
+#include "common.inc"
 
 namespace {
-
-constexpr int kS = 4;        // cell side
-constexpr int kK = kS * kS;  // taps per cell
-constexpr int kBlock = 256;  // threads per block of the cell kernels
-
-// ---------------------------------------------------------------------------
-// Element formats
-// ---------------------------------------------------------------------------
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-
-template <int DT>
-struct Fmt {
-  static constexpr int bytes = DT == LTHC_F32 ? 4 : 2;
-};
-
-template <int DT>
-LTHC_DEV float widen1(uint32_t h16) {
-  if constexpr (DT == LTHC_BF16) return __uint_as_float(h16 << 16);
-  else return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h16)));
-}
-
-template <int DT>
-LTHC_DEV void unpack2(uint32_t w, float& a, float& b) {
-  if constexpr (DT == LTHC_BF16) {
-    a = __uint_as_float(w << 16);
-    b = __uint_as_float(w & 0xffff0000u);
-  } else {
-    const f16x2_t h = __builtin_bit_cast(f16x2_t, w);
-    a = static_cast<float>(h.x);
-    b = static_cast<float>(h.y);
-  }
-}
-
-// Round-to-nearest-even narrowing (v_cvt_pk_bf16_f32 / v_cvt_f16_f32).
-template <int DT>
-LTHC_DEV uint32_t pack2(float a, float b) {
-  if constexpr (DT == LTHC_BF16) {
-    const bf16x2_t r = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
-    return __builtin_bit_cast(uint32_t, r);
-  } else {
-    const f16x2_t r = {static_cast<_Float16>(a), static_cast<_Float16>(b)};
-    return __builtin_bit_cast(uint32_t, r);
-  }
-}
-
-// Narrowing of one value to a 16-bit format (round to nearest even), bits in the low half.
-template <int DT>
-LTHC_DEV uint32_t narrow1(float v) {
-  if constexpr (DT == LTHC_BF16) return __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));
-  else return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
-}
-
-// Raw storage of N consecutive elements of format DT: whole dwords, or one
-// 16-bit element (kBytes == 2, held in the low half of w[0]).
-template <int DT, int N>
-struct Raw {
-  static constexpr int kBytes = N * Fmt<DT>::bytes;
-  static constexpr int kWords = kBytes >= 4 ? kBytes / 4 : 1;
-  static_assert(kBytes == 2 || kWords <= 2 || kWords % 4 == 0, "raw vector width");
-  uint32_t w[kWords];
-};
-
-// One vector load (dwordx1/x2/x4, several x4 for wider runs) of the raw
-// bytes at base + boff; NT = streaming (non-temporal).  With a uniform base
-// and a 32-bit offset (Off = uint32_t) this is the saddr + voffset form, so
-// the per-lane address costs one VGPR and no 64-bit arithmetic.
-template <int DT, int N, bool NT = false, typename Off = int64_t>
-LTHC_DEV void load_at(const void* __restrict__ base, Off boff, Raw<DT, N>& r) {
-  constexpr int W = Raw<DT, N>::kWords;
-  const char* q = static_cast<const char*>(base) + boff;
-  if constexpr (Raw<DT, N>::kBytes == 2) {
-    r.w[0] = NT ? __builtin_nontemporal_load(reinterpret_cast<const uint16_t*>(q)) : *reinterpret_cast<const uint16_t*>(q);
-  } else if constexpr (W == 1) {
-    r.w[0] = NT ? __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(q)) : *reinterpret_cast<const uint32_t*>(q);
-  } else if constexpr (W == 2) {
-    const u32x2_t t = NT ? __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(q)) : *reinterpret_cast<const u32x2_t*>(q);
-    r.w[0] = t.x;
-    r.w[1] = t.y;
-  } else {
-#pragma unroll
-    for (int j = 0; j < W / 4; ++j) {
-      const u32x4_t* v = reinterpret_cast<const u32x4_t*>(q) + j;
-      const u32x4_t t = NT ? __builtin_nontemporal_load(v) : *v;
-      r.w[4 * j + 0] = t.x;
-      r.w[4 * j + 1] = t.y;
-      r.w[4 * j + 2] = t.z;
-      r.w[4 * j + 3] = t.w;
-    }
-  }
-}
-
-// Element-index form.
-template <int DT, int N, bool NT = false>
-LTHC_DEV void load_raw(const void* __restrict__ p, int64_t i, Raw<DT, N>& r) {
-  load_at<DT, N, NT>(p, i * Fmt<DT>::bytes, r);
-}
-
-template <int DT, int N>
-LTHC_DEV void unpack_raw(const Raw<DT, N>& r, float (&v)[N]) {
-  if constexpr (DT == LTHC_F32) {
-#pragma unroll
-    for (int j = 0; j < N; ++j) v[j] = __uint_as_float(r.w[j]);
-  } else if constexpr (N == 1) {
-    v[0] = widen1<DT>(r.w[0]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < N / 2; ++j) unpack2<DT>(r.w[j], v[2 * j], v[2 * j + 1]);
-  }
-}
-
-template <int DT, int N>
-LTHC_DEV void load_vec(const void* __restrict__ p, int64_t i, float (&v)[N]) {
-  Raw<DT, N> r;
-  load_raw<DT, N>(p, i, r);
-  unpack_raw<DT, N>(r, v);
-}
-
-template <int DT, int N, bool NT = false, typename Off = int64_t>
-LTHC_DEV void store_at(void* __restrict__ base, Off boff, const float (&v)[N]) {
-  char* q = static_cast<char*>(base) + boff;
-  if constexpr (N * Fmt<DT>::bytes == 2) {
-    const uint16_t h = static_cast<uint16_t>(narrow1<DT>(v[0]));
-    if (NT) __builtin_nontemporal_store(h, reinterpret_cast<uint16_t*>(q));
-    else *reinterpret_cast<uint16_t*>(q) = h;
-  } else {
-    constexpr int W = N * Fmt<DT>::bytes / 4;
-    uint32_t w[W];
-    if constexpr (DT == LTHC_F32) {
-#pragma unroll
-      for (int j = 0; j < N; ++j) w[j] = __float_as_uint(v[j]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < N / 2; ++j) w[j] = pack2<DT>(v[2 * j], v[2 * j + 1]);
-    }
-    if constexpr (W == 1) {
-      if (NT) __builtin_nontemporal_store(w[0], reinterpret_cast<uint32_t*>(q));
-      else *reinterpret_cast<uint32_t*>(q) = w[0];
-    } else if constexpr (W == 2) {
-      const u32x2_t t = {w[0], w[1]};
-      if (NT) __builtin_nontemporal_store(t, reinterpret_cast<u32x2_t*>(q));
-      else *reinterpret_cast<u32x2_t*>(q) = t;
-    } else {
-      static_assert(W % 4 == 0, "store width");
-#pragma unroll
-      for (int j = 0; j < W / 4; ++j) {
-        const u32x4_t t = {w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]};
-        if (NT) __builtin_nontemporal_store(t, reinterpret_cast<u32x4_t*>(q) + j);
-        else reinterpret_cast<u32x4_t*>(q)[j] = t;
-      }
-    }
-  }
-}
-
-template <int DT, int N, bool NT = false>
-LTHC_DEV void store_vec(void* __restrict__ p, int64_t i, const float (&v)[N]) {
-  store_at<DT, N, NT>(p, i * Fmt<DT>::bytes, v);
-}
-
-// N consecutive weights of format WDT, widened to fp32 (one vector load
-// where the width allows it).
-template <int WDT, int N>
-LTHC_DEV void load_wvec(const void* __restrict__ p, int64_t i, float (&v)[N]) {
-  if constexpr (WDT == LTHC_F32 || N % 2 == 0) {
-    load_vec<WDT, N>(p, i, v);
-  } else {
-#pragma unroll
-    for (int j = 0; j < N; ++j) v[j] = widen1<WDT>(static_cast<const uint16_t*>(p)[i + j]);
-  }
-}
-
-// Scalar weight of a runtime dtype (small kernels only).
-LTHC_DEV float load_w(const void* __restrict__ p, int dt, int64_t i) {
-  if (dt == LTHC_F32) return static_cast<const float*>(p)[i];
-  const uint16_t h = static_cast<const uint16_t*>(p)[i];
-  if (dt == LTHC_BF16) return widen1<LTHC_BF16>(h);
-  return widen1<LTHC_F16>(h);
-}
-
-// Round one value to format DT (round to nearest even; identity for fp32).
-template <int DT>
-LTHC_DEV float round_w(float v) {
-  if constexpr (DT == LTHC_F32) return v;
-  else if constexpr (DT == LTHC_BF16) return static_cast<float>(static_cast<__bf16>(v));
-  else return static_cast<float>(static_cast<_Float16>(v));
-}
-
-// fp16 outputs of an fma chain are rounded once from the fp32 result: the empty asm keeps the compiler from folding
-// the last fma and the narrowing into a mixed-precision fma (one rounding of the exact value) for some lanes or
-// kernels and not others, so every kernel producing the same quantity gives the same bits.
-template <int DT, int N>
-LTHC_DEV void hold_f32(float (&v)[N]) {
-  if constexpr (DT == LTHC_F16) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
-  }
-}
-
-LTHC_DEV void store_w(void* __restrict__ p, int dt, int64_t i, float v) {
-  if (dt == LTHC_F32) {
-    static_cast<float*>(p)[i] = v;
-  } else if (dt == LTHC_BF16) {
-    static_cast<__bf16*>(p)[i] = static_cast<__bf16>(v);
-  } else {
-    static_cast<_Float16*>(p)[i] = static_cast<_Float16>(v);
-  }
-}
-
-struct PtrPack {
-  const void* p[LTHC_MAX_LAYERS];
-};
 
 // Walks consecutive cells without divisions.  hoff = element offset of tap
 // (0, 0), channel 0 of the current cell in the NHWC tensor; zoff = cell * C.
@@ -981,92 +755,6 @@ __global__ __launch_bounds__(kBlock) void cell_wgrad_kernel(const void* __restri
   }
 }
 
-__global__ __launch_bounds__(256) void zero_kernel(float* __restrict__ out, int64_t n) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i < n) out[i] = 0.f;
-}
-
-// Stage 2: out[i] = sum_{p < nparts} partial[p, i] in ascending p, stored in
-// format odt (the fp32 sum rounded once).
-__global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ partial, int nparts,
-                                                              int64_t n, void* __restrict__ out, int odt) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.f;
-  for (int p = 0; p < nparts; ++p) s += partial[static_cast<int64_t>(p) * n + i];
-  store_w(out, odt, i, s);
-}
-
-// Narrow outputs (few columns, many partial rows): block = 16 columns x 16
-// part groups; group g sums parts g, g + 16, g + 32, ... in order, then the
-// 16 group sums are added in order g = 0..15 -- a fixed order, so the result
-// is bitwise reproducible, with 16x the parallelism of reduce_partials_kernel.
-constexpr int kRedGroups = 16;
-// A 256-thread block reduces COLS consecutive columns with 256 / COLS part groups: group g sums parts g, g + NG,
-// g + 2 NG, ... in order (NG = 256 / COLS), then the group sums are added in order g = 0..NG-1.  COLS = 16 gives 16
-// groups (narrow outputs: many partial rows over few columns); COLS = 64 makes a wavefront's load one 256-byte run
-// of a partial row (wide outputs).
-template <int COLS>
-__device__ __forceinline__ void reduce_split_block(const float* __restrict__ partial, int nparts, int64_t n,
-                                                   int64_t cblock, void* __restrict__ out, int odt) {
-  constexpr int NG = 256 / COLS;
-  __shared__ float part[NG][COLS];
-  const int col = threadIdx.x % COLS;
-  const int grp = threadIdx.x / COLS;
-  const int64_t i = cblock * COLS + col;
-  float s = 0.f;
-  if (i < n) {
-    // loads in batches of 8 (in flight together), added in part order
-    int p = grp;
-    for (; p + 7 * NG < nparts; p += 8 * NG) {
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = partial[static_cast<int64_t>(p + j * NG) * n + i];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) s += v[j];
-    }
-    for (; p < nparts; p += NG) s += partial[static_cast<int64_t>(p) * n + i];
-  }
-  part[grp][col] = s;
-  __syncthreads();
-  if (grp == 0 && i < n) {
-    float t = 0.f;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) t += part[g][col];
-    store_w(out, odt, i, t);
-  }
-}
-
-template <int COLS>
-__global__ __launch_bounds__(256) void reduce_partials_split_kernel(const float* __restrict__ partial, int nparts,
-                                                                    int64_t n, void* __restrict__ out, int odt) {
-  reduce_split_block<COLS>(partial, nparts, n, blockIdx.x, out, odt);
-}
-
-// Several independent reductions in one launch (fp32 outputs), each segment's columns summed as
-// reduce_partials_split_kernel<16> sums them (16-column blocks: the 64-column form measured slower here, where
-// the segments have few partial rows).
-struct RedSeg {
-  const float* partial;
-  float* out;
-  int64_t n;
-  int64_t block0;  // first block of the segment
-  int nparts;
-};
-constexpr int kRedMaxSegs = 4;
-struct RedSegs {
-  RedSeg s[kRedMaxSegs];
-  int nseg;
-};
-
-__global__ __launch_bounds__(256) void reduce_partials_multi_kernel(RedSegs segs) {
-  const int64_t b = blockIdx.x;
-  int si = 0;
-  while (si + 1 < segs.nseg && b >= segs.s[si + 1].block0) ++si;
-  const RedSeg& sg = segs.s[si];
-  reduce_split_block<16>(sg.partial, sg.nparts, sg.n, b - sg.block0, sg.out, LTHC_F32);
-}
-
 // ---------------------------------------------------------------------------
 // GAMMA: gamma[l, c] = sum_k alpha[c,k] beta_l[c,k], k = 0..K-1 in order
 // ---------------------------------------------------------------------------
@@ -1367,35 +1055,6 @@ __global__ __launch_bounds__(256) void recur_bwd_kernel(const void* __restrict__
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
-thread_local std::string g_last_error;
-
-int fail(int code, const char* fn, const std::string& msg) {
-  g_last_error = std::string(fn) + ": " + msg;
-  return code;
-}
-
-int check_launch(const char* fn) {
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(LTHC_ERR_HIP, fn, std::string("kernel launch failed: ") + hipGetErrorString(e));
-  return LTHC_OK;
-}
-
-int num_cus() {
-  static int cache[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cache[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cache[dev] = n;
-  }
-  return cache[dev];
-}
-
-bool valid_dtype(int dt) { return dt == LTHC_F32 || dt == LTHC_BF16 || dt == LTHC_F16; }
-int esize(int dt) { return dt == LTHC_F32 ? 4 : 2; }
-bool aligned(const void* p, int64_t bytes) { return (reinterpret_cast<uintptr_t>(p) % bytes) == 0; }
-
 int check_geom(const char* fn, int64_t B, int64_t G, int64_t s, int64_t C) {
   if (B < 0) return fail(LTHC_ERR_INVALID, fn, "B must be >= 0");
   if (G <= 0 || C <= 0) return fail(LTHC_ERR_INVALID, fn, "G and C must be positive");
@@ -1403,12 +1062,6 @@ int check_geom(const char* fn, int64_t B, int64_t G, int64_t s, int64_t C) {
   if (C % 4 != 0) return fail(LTHC_ERR_INVALID, fn, "C must be a multiple of 4");
   if (G > 4096 || C > (1 << 24)) return fail(LTHC_ERR_INVALID, fn, "G or C out of range");
   if (B > (int64_t(1) << 40) / (G * G * kK * C)) return fail(LTHC_ERR_INVALID, fn, "tensor too large");
-  return LTHC_OK;
-}
-
-int check_act(const char* fn, const void* p, int dt, const char* name) {
-  if (p == nullptr) return fail(LTHC_ERR_INVALID, fn, std::string(name) + " is NULL");
-  if (!aligned(p, 4 * esize(dt))) return fail(LTHC_ERR_INVALID, fn, std::string(name) + " is not aligned to 4 elements");
   return LTHC_OK;
 }
 
@@ -1479,38 +1132,6 @@ const int64_t kRecurBwdChunks = 256;
 
 int64_t recur_bwd_blocks_y(int64_t rows) { return std::min((rows + 4 * kRUB - 1) / (4 * kRUB), kRecurBwdChunks); }
 
-// Deterministic reduction of nparts partial rows of n floats into out.
-void launch_reduce(const float* partial, int nparts, int64_t n, void* out, hipStream_t st, int odt = LTHC_F32) {
-  if (nparts <= kRedGroups) {
-    reduce_partials_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, st>>>(partial, nparts, n, out, odt);
-  } else if (n >= 64 * 256) {  // wide: 64-column blocks (a wavefront's load is one 256-byte run of a partial row)
-    reduce_partials_split_kernel<64><<<static_cast<unsigned>((n + 63) / 64), 256, 0, st>>>(partial, nparts, n, out, odt);
-  } else {
-    reduce_partials_split_kernel<16><<<static_cast<unsigned>((n + 15) / 16), 256, 0, st>>>(partial, nparts, n, out, odt);
-  }
-}
-
-// The reductions of up to kRedMaxSegs (partial, nparts, n, out) segments in one launch.
-void launch_reduce_multi(std::initializer_list<RedSeg> list, hipStream_t st) {
-  RedSegs segs{};
-  int64_t blocks = 0;
-  for (const RedSeg& r : list) {
-    RedSeg& d = segs.s[segs.nseg++];
-    d = r;
-    d.block0 = blocks;
-    blocks += (r.n + 15) / 16;
-  }
-  reduce_partials_multi_kernel<<<static_cast<unsigned>(blocks), 256, 0, st>>>(segs);
-}
-
-template <int V>
-using IC = std::integral_constant<int, V>;
-
-template <typename T>
-struct TypeTag {
-  using type = T;
-};
-
 // Calls f(IC<DT>, IC<WDT>) for a supported (activation, weight) dtype pair.
 template <typename F>
 void dispatch_pair(int xdt, int wdt, F&& f) {
@@ -1524,15 +1145,6 @@ void dispatch_pair(int xdt, int wdt, F&& f) {
       if (wdt == LTHC_F32) f(IC<LTHC_F16>{}, IC<LTHC_F32>{});
       else f(IC<LTHC_F16>{}, IC<LTHC_F16>{});
       break;
-  }
-}
-
-template <typename F>
-void dispatch_dtype(int dt, F&& f) {
-  switch (dt) {
-    case LTHC_F32: f(IC<LTHC_F32>{}); break;
-    case LTHC_BF16: f(IC<LTHC_BF16>{}); break;
-    default: f(IC<LTHC_F16>{}); break;
   }
 }
 
@@ -2232,14 +1844,8 @@ int lthc_recur_bwd_sum(const void* g, const void* g_branch, const void* dz, cons
 
 }  // extern "C"
 
-// Final-layer RMSNorm + modulate of the decoder input (the materialisation's consumer).
-#include "norm_modulate.inc"
-
 // Workspace accumulation of the non-shared (triangular lazy) interface.
 #include "ws_accumulate.inc"
-#include "branch_ops.inc"
-// Fused q/k RMSNorm + RoPE and attention of the branch (matrix cores).
-#include "attention.inc"
 // The decoder head (norm + modulate + linear + unpatchify) on the matrix cores.
 #include "decoder.inc"
 // One-launch dtype conversion of many weights (autocast's per-forward casts).
