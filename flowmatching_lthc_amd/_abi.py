@@ -50,6 +50,8 @@ EXPORTS = (
     "lthc_norm_modulate_bwd",
     "lthc_qk_norm_rope",
     "lthc_qk_norm_rope_attention",
+    "lthc_qk_norm_rope_attention_bwd_workspace_bytes",
+    "lthc_qk_norm_rope_attention_bwd",
     "lthc_decoder_fwd",
     "lthc_materialise_decoder_workspace_bytes",
     "lthc_materialise_decoder_fwd",
@@ -110,6 +112,10 @@ def load() -> ctypes.CDLL:
         "lthc_qk_norm_rope_attention": [
             vp, ci, vp, vp, ci, vp, vp, ci, vp, i64, i64, i64, i64, ctypes.c_float, ctypes.c_float, vp,
         ],  # fmt: skip
+        "lthc_qk_norm_rope_attention_bwd": [
+            vp, vp, ci, vp, vp, ci, vp, vp, ci, vp, vp, ci, i64, i64, i64, i64, ctypes.c_float, ctypes.c_float, vp, sz,
+            vp,
+        ],  # fmt: skip
         "lthc_decoder_fwd": [
             vp, ci, vp, ci, vp, vp, i64, vp, ci, vp, ci, vp, i64, i64, i64, i64, i64, i64, ctypes.c_float, vp,
         ],  # fmt: skip
@@ -156,6 +162,8 @@ def load() -> ctypes.CDLL:
     lib.lthc_ws_accumulate_bwd_workspace_bytes.restype = sz
     lib.lthc_norm_modulate_bwd_workspace_bytes.argtypes = [i64, i64, i64]
     lib.lthc_norm_modulate_bwd_workspace_bytes.restype = sz
+    lib.lthc_qk_norm_rope_attention_bwd_workspace_bytes.argtypes = [i64, i64, i64, i64]
+    lib.lthc_qk_norm_rope_attention_bwd_workspace_bytes.restype = sz
     _lib = lib
     return lib
 

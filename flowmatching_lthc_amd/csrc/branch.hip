@@ -9,3 +9,5 @@
 #include "branch_ops.inc"
 // Fused q/k RMSNorm + RoPE and attention of the branch (matrix cores).
 #include "attention.inc"
+// Its backward.
+#include "attention_backward.inc"

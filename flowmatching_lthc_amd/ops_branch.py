@@ -35,7 +35,6 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 from torch import Tensor
-from torch._subclasses.fake_tensor import is_fake
 
 from . import _abi
 from .ops import _fake, _mod_rows, _norm_weight, _on_device, _on_gpu
@@ -91,19 +90,24 @@ def _check_qk(qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos: Tensor, sin:
     return b, n, h
 
 
+def _qk_operands(qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos: Tensor, sin: Tensor) -> tuple[Tensor, ...]:
+    """(q weight, k weight, cos, sin) as the kernels take them: fp32 or the activation dtype (bf16 parameters and
+    buffers are used as they are), each pair in one dtype, aligned."""
+    qw, kw, c, s = (t if t.dtype == qkv.dtype else t.float() for t in (q_weight, k_weight, cos, sin))
+    if kw.dtype != qw.dtype:
+        qw, kw = qw.float(), kw.float()
+    if s.dtype != c.dtype:
+        c, s = c.float(), s.float()
+    return _aligned(qw), _aligned(kw), _aligned(c), _aligned(s)
+
+
 @torch.library.custom_op("jit_thc::qk_norm_rope", mutates_args=())
 def qk_norm_rope(qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos: Tensor, sin: Tensor, eps: float) -> tuple[Tensor, Tensor]:
     """(rope(RMSNorm_q(q)), rope(RMSNorm_k(k))) as [B, N, H, 64] in qkv's dtype, one pass over q and k."""
     _on_gpu(qkv, q_weight, k_weight, cos, sin)
     b, n, h = _check_qk(qkv, q_weight, k_weight, cos, sin)
     qkv = _aligned(qkv)
-    # weights and tables: fp32 or the activation dtype (bf16 parameters and buffers are used as they are)
-    qw, kw, c, s = (t if t.dtype == qkv.dtype else t.float() for t in (q_weight, k_weight, cos, sin))
-    if kw.dtype != qw.dtype:
-        qw, kw = qw.float(), kw.float()
-    if s.dtype != c.dtype:
-        c, s = c.float(), s.float()
-    qw, kw, c, s = (_aligned(t) for t in (qw, kw, c, s))
+    qw, kw, c, s = _qk_operands(qkv, q_weight, k_weight, cos, sin)
     q = torch.empty((b, n, h, QK_HEAD_DIM), device=qkv.device, dtype=qkv.dtype)
     k = torch.empty_like(q)
     with _on_device(qkv):
@@ -187,12 +191,7 @@ def qk_norm_rope_attention(qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos:
         raise ValueError(f"qkv must be bf16 or fp16 [B,N,3,H,64] with N a multiple of 64 up to {ATTN_MAX_TOKENS}, got "
                          f"{tuple(qkv.shape)} {qkv.dtype}")
     qkv = _aligned(qkv)
-    qw, kw, c, s = (t if t.dtype == qkv.dtype else t.float() for t in (q_weight, k_weight, cos, sin))
-    if kw.dtype != qw.dtype:
-        qw, kw = qw.float(), kw.float()
-    if s.dtype != c.dtype:
-        c, s = c.float(), s.float()
-    qw, kw, c, s = (_aligned(t) for t in (qw, kw, c, s))
+    qw, kw, c, s = _qk_operands(qkv, q_weight, k_weight, cos, sin)
     out = torch.empty((b, n, h, QK_HEAD_DIM), device=qkv.device, dtype=qkv.dtype)
     with _on_device(qkv):
         rc = _abi.load().lthc_qk_norm_rope_attention(
@@ -209,33 +208,56 @@ def _(qkv, q_weight, k_weight, cos, sin, eps):
     return qkv.new_empty((b, n, h, d))
 
 
-def _attention_fp32_recompute(qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos: Tensor, sin: Tensor, eps: float):
-    """qk_norm_rope_attention_eager's function with the attention itself in fp32 matrix products and softmax
-    (softmax(q k^T / sqrt(64)) v, rounded once to qkv's dtype): the backward's recompute when torch.compile traces it.
-    Plain products, not the SDPA kernels: the ROCm flash-attention backward returns gradient strides its meta function
-    does not predict, which compiled graphs assert on.  Eager backwards keep the SDPA recompute (at B=64 the fp32
-    products made the LTHC-B/4 training step 25 % slower)."""
-    q, k = qk_norm_rope_eager(qkv, q_weight, k_weight, cos, sin, eps)
-    v = qkv[:, :, 2]
-    q, k, v = (t.transpose(1, 2).float().contiguous() for t in (q, k, v))
-    kt = k.transpose(-1, -2).contiguous()
-    p = torch.softmax(torch.matmul(q, kt) * (QK_HEAD_DIM**-0.5), dim=-1)
-    return torch.matmul(p, v).to(qkv.dtype).transpose(1, 2)
+@torch.library.custom_op("jit_thc::qk_norm_rope_attention_backward", mutates_args=())
+def qk_norm_rope_attention_backward(
+    grad: Tensor, qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos: Tensor, sin: Tensor, eps: float
+) -> tuple[Tensor, Tensor]:
+    """(gradient of qkv in qkv's dtype, fp32 [2, 64] gradients of the q and k norm weights) of
+    qk_norm_rope_attention for the output gradient `grad` [B, N, H, 64], one matrix-core pass over qkv and grad."""
+    _on_gpu(qkv, grad, q_weight, k_weight, cos, sin)
+    b, n, h = _check_qk(qkv, q_weight, k_weight, cos, sin)
+    if not attention_supported(qkv) or tuple(grad.shape) != (b, n, h, QK_HEAD_DIM):
+        raise ValueError(f"unsupported qkv {tuple(qkv.shape)} {qkv.dtype} or grad {tuple(grad.shape)}")
+    qkv, grad = _aligned(qkv), _aligned(grad.to(qkv.dtype))
+    qw, kw, c, s = _qk_operands(qkv, q_weight, k_weight, cos, sin)
+    dqkv = torch.empty_like(qkv)
+    dw = torch.empty((2, QK_HEAD_DIM), device=qkv.device, dtype=torch.float32)
+    lib = _abi.load()
+    nbytes = int(lib.lthc_qk_norm_rope_attention_bwd_workspace_bytes(b, n, h, QK_HEAD_DIM))
+    ws = torch.empty((max(nbytes, 16),), device=qkv.device, dtype=torch.uint8)
+    with _on_device(qkv):
+        rc = lib.lthc_qk_norm_rope_attention_bwd(
+            qkv.data_ptr(), grad.data_ptr(), _abi.code(qkv), qw.data_ptr(), kw.data_ptr(), _abi.code(qw), c.data_ptr(),
+            s.data_ptr(), _abi.code(c), dqkv.data_ptr(), dw.data_ptr(), _abi.F32, b, n, h, QK_HEAD_DIM, eps,
+            QK_HEAD_DIM**-0.5, ws.data_ptr(), ws.numel(), _abi.stream_of(qkv),
+        )  # fmt: skip
+    _abi.check(rc, "lthc_qk_norm_rope_attention_bwd")
+    return dqkv, dw
 
 
-def _traced(t: Tensor) -> bool:
-    """True while torch.compile traces the code (Dynamo, or AOTAutograd on fake tensors), False when it runs."""
-    return torch.compiler.is_compiling() or is_fake(t)
+@_fake(qk_norm_rope_attention_backward)
+def _(grad, qkv, q_weight, k_weight, cos, sin, eps):
+    return torch.empty_like(qkv), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
+
+
+def _batched(*grads: Tensor | None) -> bool:
+    """A gradient is a vmap batch (autograd.grad(..., is_grads_batched=True), functorch): the backward kernels take
+    one gradient, so the eager sequence, which vmap maps op by op, is differentiated instead."""
+    return any(g is not None and torch._C._functorch.is_batchedtensor(g) for g in grads)
 
 
 def _backward_qk_attention(ctx, grad):
     qkv, q_weight, k_weight, cos, sin = ctx.saved_tensors
     need = ctx.needs_input_grad
-    # eager: the SDPA recompute (flash / efficient kernels); traced: fp32 products, whose strides the graph predicts
-    recompute = _attention_fp32_recompute if _traced(grad) else qk_norm_rope_attention_eager
+    if not _batched(grad):
+        with torch.no_grad():
+            dqkv, dw = qk_norm_rope_attention_backward(grad, qkv, q_weight, k_weight, cos, sin, ctx.eps)
+            dq = dw[0].to(q_weight.dtype) if need[1] else None
+            dk = dw[1].to(k_weight.dtype) if need[2] else None
+        return dqkv if need[0] else None, dq, dk, None, None, None
     with torch.enable_grad():
         leaves = [t.detach().requires_grad_(bool(r)) for t, r in zip((qkv, q_weight, k_weight), need[:3])]
-        o = recompute(leaves[0], leaves[1], leaves[2], cos, sin, ctx.eps)
+        o = qk_norm_rope_attention_eager(leaves[0], leaves[1], leaves[2], cos, sin, ctx.eps)
         wanted = [t for t in leaves if t.requires_grad]
         got = torch.autograd.grad([o], wanted, [grad], allow_unused=True) if wanted else []
     it = iter(got)

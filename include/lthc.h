@@ -332,6 +332,23 @@ int lthc_qk_norm_rope_attention(const void* qkv, int x_dtype, const void* q_weig
                                 int64_t N, int64_t H, int64_t D, float eps, float scale, void* stream);
 
 /*
+ * BACKWARD of lthc_qk_norm_rope_attention (autograd of local_thc.py:246-251):
+ * grad [B, N, H, D] (x_dtype) is the gradient of out; dqkv [B, N, 3, H, D]
+ * (x_dtype) receives the gradients of q, k and v, dweights [2, D] (dw_dtype)
+ * those of the q and k norm weights, reduced in a fixed order.  The forward's
+ * q_n, k_n and probabilities are recomputed; the probabilities and the score
+ * gradients are rounded to x_dtype where they enter a product, everything
+ * else is fp32 and rounded once.  Shapes, dtypes and alignment as the
+ * forward; grad and dqkv 16-byte aligned.
+ */
+size_t lthc_qk_norm_rope_attention_bwd_workspace_bytes(int64_t B, int64_t N, int64_t H, int64_t D);
+int lthc_qk_norm_rope_attention_bwd(const void* qkv, const void* grad, int x_dtype, const void* q_weight,
+                                    const void* k_weight, int w_dtype, const void* cos_table, const void* sin_table,
+                                    int table_dtype, void* dqkv, void* dweights, int dw_dtype, int64_t B, int64_t N,
+                                    int64_t H, int64_t D, float eps, float scale, void* workspace,
+                                    size_t workspace_bytes, void* stream);
+
+/*
  * DECODER HEAD (no reference op: FinalLayerSharedAdaLN.forward and
  * unpatchify, local_thc.py:865-873 and :972-980, are eager torch).  For the
  * materialised x [B, h*w, C] (x_dtype bf16 or fp16):
