@@ -58,7 +58,11 @@ EXPORTS = (
     "lthc_cast_many",
     "lthc_swiglu",
     "lthc_gate_add_norm_modulate_fwd",
+    "lthc_gate_add_norm_modulate_bwd_workspace_bytes",
+    "lthc_gate_add_norm_modulate_bwd",
     "lthc_gate_residual",
+    "lthc_gate_residual_bwd_workspace_bytes",
+    "lthc_gate_residual_bwd",
     "lthc_block_tail_fwd",
     "lthc_recur_fwd_prefix",
     "lthc_read_bwd_workspace_bytes",
@@ -125,6 +129,11 @@ def load() -> ctypes.CDLL:
         ],  # fmt: skip
         "lthc_cast_many": [vp, vp, i64, vp, ci, vp],
         "lthc_swiglu": [vp, ci, vp, i64, i64, vp],
+        "lthc_gate_add_norm_modulate_bwd": [
+            vp, vp, vp, vp, vp, ci, vp, ci, vp, i64, vp, vp, vp, vp, vp, vp, ci, i64, i64, i64, ctypes.c_float, vp, sz,
+            vp,
+        ],  # fmt: skip
+        "lthc_gate_residual_bwd": [vp, vp, vp, i64, ci, vp, vp, i64, i64, i64, vp, sz, vp],
         "lthc_gate_add_norm_modulate_fwd": [
             vp, vp, vp, ci, vp, ci, vp, vp, i64, vp, vp, vp, i64, i64, i64, ctypes.c_float, vp,
         ],  # fmt: skip
@@ -162,8 +171,14 @@ def load() -> ctypes.CDLL:
     lib.lthc_ws_accumulate_bwd_workspace_bytes.restype = sz
     lib.lthc_norm_modulate_bwd_workspace_bytes.argtypes = [i64, i64, i64]
     lib.lthc_norm_modulate_bwd_workspace_bytes.restype = sz
-    lib.lthc_qk_norm_rope_attention_bwd_workspace_bytes.argtypes = [i64, i64, i64, i64]
-    lib.lthc_qk_norm_rope_attention_bwd_workspace_bytes.restype = sz
+    for name in ("lthc_qk_norm_rope_attention_bwd",):
+        fn = getattr(lib, name + "_workspace_bytes")
+        fn.argtypes = [i64, i64, i64, i64]
+        fn.restype = sz
+    for name in ("lthc_gate_add_norm_modulate_bwd", "lthc_gate_residual_bwd"):
+        fn = getattr(lib, name + "_workspace_bytes")
+        fn.argtypes = [i64, i64, i64]
+        fn.restype = sz
     _lib = lib
     return lib
 

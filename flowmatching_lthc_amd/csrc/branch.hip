@@ -7,7 +7,9 @@
 // RMSNorm + modulate (the decoder's input and the branch's pre-norms) with its gated forms.
 #include "norm_modulate.inc"
 #include "branch_ops.inc"
+// Backward of the elementwise ops.
+#include "branch_backward.inc"
 // Fused q/k RMSNorm + RoPE and attention of the branch (matrix cores).
 #include "attention.inc"
-// Its backward.
+// The attention's backward.
 #include "attention_backward.inc"

@@ -24,10 +24,10 @@ activation dtype), registered as a ``jit_thc`` custom op:
   and the next block's first pre-norm (:315-317) in one pass, each value
   that of the three separate ops.
 
-The backward of all but gate_residual recomputes the eager sequence under
-autograd (the forward's values are those of that sequence; the attention's
-products accumulate in fp32 as SDPA's do), so training through them matches
-the eager model's gradients; gate_residual's is its closed form.
+Every op but block_tail (inference only) has a backward kernel of its own,
+``jit_thc::<op>_backward``, one HIP pass that recomputes what it needs from the
+op's inputs and gives the gradients of the eager sequence.  Batched gradients
+(vmap) differentiate the eager sequence itself.
 """
 
 from __future__ import annotations
@@ -37,13 +37,13 @@ import torch.nn.functional as F
 from torch import Tensor
 
 from . import _abi
-from .ops import _fake, _mod_rows, _norm_weight, _on_device, _on_gpu
+from .ops import _fake, _mod_rows, _norm_weight, _on_device, _on_gpu, _prep
 
 QK_HEAD_DIM = 64
 
 
 # ---------------------------------------------------------------------------
-# eager restatements (the backward recomputes these)
+# eager restatements (the tests' reference; batched gradients differentiate them)
 # ---------------------------------------------------------------------------
 def _rms_norm_eager(x: Tensor, weight: Tensor, eps: float) -> Tensor:
     xf = x.float()
@@ -73,6 +73,16 @@ def _aligned(t: Tensor) -> Tensor:
     """Contiguous with a 16-byte aligned start (the kernels use 16-byte vector accesses)."""
     t = t.contiguous()
     return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _batched(*grads: Tensor | None) -> bool:
+    """A gradient is a vmap batch (autograd.grad(..., is_grads_batched=True), functorch): the backward kernels take
+    one gradient, so the eager sequence, which vmap maps op by op, is differentiated instead."""
+    return any(g is not None and torch._C._functorch.is_batchedtensor(g) for g in grads)
+
+
+def _workspace(nbytes: int, like: Tensor) -> Tensor:
+    return torch.empty((max(int(nbytes), 16),), device=like.device, dtype=torch.uint8)
 
 
 # ---------------------------------------------------------------------------
@@ -223,8 +233,7 @@ def qk_norm_rope_attention_backward(
     dqkv = torch.empty_like(qkv)
     dw = torch.empty((2, QK_HEAD_DIM), device=qkv.device, dtype=torch.float32)
     lib = _abi.load()
-    nbytes = int(lib.lthc_qk_norm_rope_attention_bwd_workspace_bytes(b, n, h, QK_HEAD_DIM))
-    ws = torch.empty((max(nbytes, 16),), device=qkv.device, dtype=torch.uint8)
+    ws = _workspace(lib.lthc_qk_norm_rope_attention_bwd_workspace_bytes(b, n, h, QK_HEAD_DIM), qkv)
     with _on_device(qkv):
         rc = lib.lthc_qk_norm_rope_attention_bwd(
             qkv.data_ptr(), grad.data_ptr(), _abi.code(qkv), qw.data_ptr(), kw.data_ptr(), _abi.code(qw), c.data_ptr(),
@@ -238,12 +247,6 @@ def qk_norm_rope_attention_backward(
 @_fake(qk_norm_rope_attention_backward)
 def _(grad, qkv, q_weight, k_weight, cos, sin, eps):
     return torch.empty_like(qkv), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
-
-
-def _batched(*grads: Tensor | None) -> bool:
-    """A gradient is a vmap batch (autograd.grad(..., is_grads_batched=True), functorch): the backward kernels take
-    one gradient, so the eager sequence, which vmap maps op by op, is differentiated instead."""
-    return any(g is not None and torch._C._functorch.is_batchedtensor(g) for g in grads)
 
 
 def _backward_qk_attention(ctx, grad):
@@ -363,6 +366,50 @@ def _(z, a, gate, weight, shift, scale, eps):
     return torch.empty_like(z), torch.empty_like(z)
 
 
+def _grad_dtype(weight: Tensor) -> torch.dtype:
+    """The dtype the kernels write a norm weight's gradient in: the weight's own where it is one of theirs."""
+    return weight.dtype if weight.dtype in _abi.DTYPE_CODE else torch.float32
+
+
+@torch.library.custom_op("jit_thc::gate_add_norm_modulate_backward", mutates_args=())
+def gate_add_norm_modulate_backward(
+    grad_d: Tensor | None, grad_y: Tensor, z: Tensor, a: Tensor, gate: Tensor, weight: Tensor, scale: Tensor, eps: float
+) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
+    """Gradients of gate_add_norm_modulate's (z, a, gate, weight, shift, scale) for those of d (None: zero) and y, one
+    pass over z, a and the gradients; the weight's in its own dtype, the others in z's."""
+    _on_gpu(z, a, gate, weight, scale, grad_y)
+    b, n, c = z.shape
+    grads = [g for g in (grad_d, grad_y) if g is not None]
+    for name, t in (("a", a), ("grad", grads[0]), ("grad", grads[-1])):
+        if tuple(t.shape) != (b, n, c):
+            raise ValueError(f"{name} must be {[b, n, c]}, got {tuple(t.shape)}")
+    z, a, grad_y = _prep(z), _prep(a), _prep(grad_y.to(z.dtype))
+    if grad_d is not None:
+        grad_d = _prep(grad_d.to(z.dtype))
+    (gate, scale), ld = _mod_rows(gate, scale)
+    w = _norm_weight(weight)
+    gz, ga = torch.empty_like(z), torch.empty_like(z)
+    ggate, gshift, gscale = (torch.empty((b, c), device=z.device, dtype=z.dtype) for _ in range(3))
+    gw = torch.empty((c,), device=z.device, dtype=_grad_dtype(weight))
+    lib = _abi.load()
+    ws = _workspace(lib.lthc_gate_add_norm_modulate_bwd_workspace_bytes(b, n, c), z)
+    with _on_device(z):
+        rc = lib.lthc_gate_add_norm_modulate_bwd(
+            _abi.ptr(grad_d), grad_y.data_ptr(), z.data_ptr(), a.data_ptr(), gate.data_ptr(), _abi.code(z), w.data_ptr(),
+            _abi.code(w), scale.data_ptr(), ld, gz.data_ptr(), ga.data_ptr(), ggate.data_ptr(), gshift.data_ptr(),
+            gscale.data_ptr(), gw.data_ptr(), _abi.code(gw), b, n, c, eps, ws.data_ptr(), ws.numel(), _abi.stream_of(z),
+        )  # fmt: skip
+    _abi.check(rc, "lthc_gate_add_norm_modulate_bwd")
+    return gz, ga, ggate, gw, gshift, gscale
+
+
+@_fake(gate_add_norm_modulate_backward)
+def _(grad_d, grad_y, z, a, gate, weight, scale, eps):
+    b, _, c = z.shape
+    row = lambda: z.new_empty((b, c))  # noqa: E731
+    return torch.empty_like(z), torch.empty_like(z), row(), z.new_empty((c,), dtype=_grad_dtype(weight)), row(), row()
+
+
 def _setup_ganm_ctx(ctx, inputs, output):
     ctx.save_for_backward(*inputs[:6])
     ctx.eps = inputs[6]
@@ -371,6 +418,11 @@ def _setup_ganm_ctx(ctx, inputs, output):
 def _backward_ganm(ctx, grad_d, grad_y):
     saved = ctx.saved_tensors
     need = ctx.needs_input_grad[:6]
+    if grad_y is not None and not _batched(grad_d, grad_y):
+        z, a, gate, weight, _, scale = saved
+        with torch.no_grad():
+            grads = gate_add_norm_modulate_backward(grad_d, grad_y, z, a, gate, weight, scale, ctx.eps)
+            return (*[g.to(t.dtype) if r else None for g, t, r in zip(grads, saved, need)], None)
     with torch.enable_grad():
         leaves = [t.detach().requires_grad_(bool(r)) for t, r in zip(saved, need)]
         d, y = gate_add_norm_modulate_eager(*leaves, ctx.eps)
@@ -411,6 +463,35 @@ def _(d, gate, m):
     return torch.empty_like(d)
 
 
+GATE_RESIDUAL_BACKWARD_MAX_CHANNELS = 2048
+
+
+@torch.library.custom_op("jit_thc::gate_residual_backward", mutates_args=())
+def gate_residual_backward(grad: Tensor, gate: Tensor, m: Tensor) -> tuple[Tensor, Tensor]:
+    """(gradient of gate [B,C], gradient of m [B,N,C]) of gate_residual in grad's dtype, one pass over grad and m."""
+    _on_gpu(grad, gate, m)
+    b, n, c = grad.shape
+    _check_bnc("m", m, (b, n, c), grad.dtype)
+    _check_bnc("gate", gate, (b, c), grad.dtype)
+    grad, m = _prep(grad), _prep(m)
+    (gate,), ld = _mod_rows(gate)
+    gm, ggate = torch.empty_like(m), torch.empty((b, c), device=m.device, dtype=m.dtype)
+    lib = _abi.load()
+    ws = _workspace(lib.lthc_gate_residual_bwd_workspace_bytes(b, n, c), m)
+    with _on_device(m):
+        rc = lib.lthc_gate_residual_bwd(
+            grad.data_ptr(), m.data_ptr(), gate.data_ptr(), ld, _abi.code(m), gm.data_ptr(), ggate.data_ptr(), b, n, c,
+            ws.data_ptr(), ws.numel(), _abi.stream_of(m),
+        )  # fmt: skip
+    _abi.check(rc, "lthc_gate_residual_bwd")
+    return ggate, gm
+
+
+@_fake(gate_residual_backward)
+def _(grad, gate, m):
+    return grad.new_empty(gate.shape), torch.empty_like(m)
+
+
 def _setup_gres_ctx(ctx, inputs, output):
     d, gate, m = inputs
     ctx.save_for_backward(gate, m)
@@ -419,6 +500,10 @@ def _setup_gres_ctx(ctx, inputs, output):
 def _backward_gres(ctx, grad):
     gate, m = ctx.saved_tensors
     need = ctx.needs_input_grad
+    if (need[1] or need[2]) and m.shape[2] <= GATE_RESIDUAL_BACKWARD_MAX_CHANNELS and not _batched(grad):
+        with torch.no_grad():
+            grad_gate, grad_m = gate_residual_backward(grad, gate, m)
+        return grad if need[0] else None, grad_gate if need[1] else None, grad_m if need[2] else None
     grad_d = grad if need[0] else None
     grad_gate = (grad * m).float().sum(1).to(gate.dtype) if need[1] else None
     grad_m = grad * gate.unsqueeze(1) if need[2] else None

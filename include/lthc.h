@@ -438,6 +438,31 @@ int lthc_gate_residual(const void* d, const void* gate, int64_t gate_ld, const v
                        int64_t B, int64_t N, int64_t C, void* stream);
 
 /*
+ * BACKWARD of lthc_gate_add_norm_modulate_fwd (autograd of
+ * local_thc.py:319-322): grad_d (NULL: zero) and grad_y are the gradients of
+ * d_out and y; gz, ga [B, N, C] and ggate, gshift, gscale [B, C] (dense) are
+ * written in x_dtype, gweight [C] in gw_dtype.  The inverse RMS is recomputed;
+ * sums are fp32 in a fixed order and each result is rounded once.
+ */
+size_t lthc_gate_add_norm_modulate_bwd_workspace_bytes(int64_t B, int64_t N, int64_t C);
+int lthc_gate_add_norm_modulate_bwd(const void* grad_d, const void* grad_y, const void* z, const void* a,
+                                    const void* gate, int x_dtype, const void* weight, int w_dtype, const void* scale,
+                                    int64_t mod_ld, void* gz, void* ga, void* ggate, void* gshift, void* gscale,
+                                    void* gweight, int gw_dtype, int64_t B, int64_t N, int64_t C, float eps,
+                                    void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * BACKWARD of lthc_gate_residual (autograd of local_thc.py:322-323): gm =
+ * r(gate * grad) [B, N, C] and ggate[b,c] = sum_n grad * m ([B, C] dense, fp32
+ * sum in a fixed order, rounded once), both x_dtype; dL/dd is grad itself.
+ * C a multiple of 4, at most 2048.
+ */
+size_t lthc_gate_residual_bwd_workspace_bytes(int64_t B, int64_t N, int64_t C);
+int lthc_gate_residual_bwd(const void* grad, const void* m, const void* gate, int64_t gate_ld, int x_dtype, void* gm,
+                           void* ggate, int64_t B, int64_t N, int64_t C, void* workspace, size_t workspace_bytes,
+                           void* stream);
+
+/*
  * BLOCK TAIL (inference): one block's last gated residual, the lazy
  * recurrence step and the next block's first pre-norm in one pass.  Per token
  * t of sample b, channel c (z = Z_l, a = the attention's gated residual

@@ -7,6 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from flowmatching_lthc_amd import ops
 from flowmatching_lthc_amd import ops_branch as OB
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +62,72 @@ def test_attention_backward(N, H, dtype, tdt, wdt):
     assert rel(gb[1], 2 * exact[0]) <= 1.1 * rel(got[1][0], exact[0])
     e, dw = OB.qk_norm_rope_attention_backward(g[:0], qkv[:0], w0, w1, cos, sin, 1e-6)
     assert e.shape == (0, N, 3, H, 64) and dw.abs().max().item() == 0.0
+
+
+UNIT = {torch.float32: 2.0**-24, torch.bfloat16: 2.0**-9, torch.float16: 2.0**-12}
+
+
+def check_grads(names, ours, eager, exact, dtype):
+    """Each gradient no further from the exact one than eager's (x 1.1) plus one rounding of the result; fp32 sums in
+    another order: 1e-6."""
+    for name, a, e, x in zip(names, ours, eager, exact):
+        assert a.dtype == e.dtype and a.shape == e.shape, name
+        bound = 1.1 * rel(e, x) + UNIT[dtype] + (1e-6 if dtype == torch.float32 else 0.0)
+        assert rel(a, x) <= bound, f"{name}: {rel(a, x):.2e}, eager {rel(e, x):.2e}"
+
+
+def grads_of(fn, tensors, outs, dtype=None):
+    leaves = [(t.to(dtype) if dtype else t.clone()).detach().requires_grad_() for t in tensors]
+    got = fn(*leaves)
+    got = got if isinstance(got, tuple) else (got,)
+    return torch.autograd.grad(got, leaves, [g.to(o.dtype) for g, o in zip(outs, got)])
+
+
+def norm_mod_exact(x, w, shift, scale):
+    n = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * w
+    return n * (1 + scale[:, None]) + shift[:, None]
+
+
+# C: below and past one 256-channel chunk, the 3-chunk form and the widest; N: one token, runs that end inside a block,
+# a sample longer than a block's run; B * N large enough for the 16-token runs (1, 8192) and larger (40, 1030)
+@pytest.mark.parametrize("B,N,C", [(2, 1, 8), (3, 9, 260), (2, 257, 768), (1, 8192, 64), (40, 1030, 128), (2, 33, 1152), (2, 5, 2048)])
+@pytest.mark.parametrize("dtype,wdt", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+def test_gated_norm_backward(B, N, C, dtype, wdt):
+    print(f"case gated norm backward B={B} N={N} C={C} {dtype} {wdt}", flush=True)
+    gen = torch.Generator().manual_seed(N + C)
+    z, a, m, gd, gy = (torch.randn((B, N, C), generator=gen).to(DEV, dtype) for _ in range(5))
+    t6 = (torch.randn((B, 3 * C), generator=gen) * 0.3).to(DEV, dtype)
+    gate, shift, scale = t6.chunk(3, -1)  # strided rows, as the model passes them
+    w = (torch.randn(C, generator=gen) * 0.1 + 1).to(DEV, wdt)
+
+    def exact(z, a, gate, w, shift, scale):
+        d = gate[:, None] * a
+        return d, norm_mod_exact(z + d, w, shift, scale)
+
+    tensors, names = (z, a, gate, w, shift, scale), ("z", "a", "gate", "weight", "shift", "scale")
+    ours = grads_of(lambda *t: OB.gate_add_norm_modulate(*t, 1e-6), tensors, (gd, gy))
+    eager = grads_of(lambda *t: OB.gate_add_norm_modulate_eager(*t, 1e-6), tensors, (gd, gy))
+    check_grads(names, ours, eager, grads_of(exact, tensors, (gd, gy), torch.float64), dtype)
+    # no gradient of d is a zero gradient of d
+    zero = OB.gate_add_norm_modulate_backward(torch.zeros_like(gd), gy, z, a, gate, w, scale, 1e-6)
+    for p, q in zip(OB.gate_add_norm_modulate_backward(None, gy, z, a, gate, w, scale, 1e-6), zero):
+        assert torch.equal(p, q)
+
+    tensors = (z, w, shift, scale)
+    ours = grads_of(lambda *t: ops.norm_modulate(*t, 1e-6)[0], tensors, (gy,))
+    eager = grads_of(lambda x, w, sh, sc: OB._rms_norm_eager(x, w, 1e-6) * (1 + sc[:, None]) + sh[:, None], tensors, (gy,))
+    check_grads(("x", "weight", "shift", "scale"), ours, eager, grads_of(norm_mod_exact, tensors, (gy,), torch.float64), dtype)
+
+    if C % 8 == 0:
+        tensors = (gd, gate, m)
+        ours, eager = grads_of(OB.gate_residual, tensors, (gy,)), grads_of(OB.gate_residual_eager, tensors, (gy,))
+        check_grads(("d", "gate", "m"), ours, eager, grads_of(OB.gate_residual_eager, tensors, (gy,), torch.float64), dtype)
+
+
+def test_gate_residual_backward_past_2048_channels():
+    print("case gate residual backward C=2056", flush=True)
+    gen = torch.Generator().manual_seed(0)
+    d, m, g = (torch.randn((2, 3, 2056), generator=gen).to(DEV, torch.bfloat16) for _ in range(3))
+    gate = torch.randn((2, 2056), generator=gen).to(DEV, torch.bfloat16)
+    ours, eager = grads_of(OB.gate_residual, (d, gate, m), (g,)), grads_of(OB.gate_residual_eager, (d, gate, m), (g,))
+    check_grads(("d", "gate", "m"), ours, eager, grads_of(OB.gate_residual_eager, (d, gate, m), (g,), torch.float64), torch.bfloat16)
