@@ -57,6 +57,7 @@ EXPORTS = (
     "lthc_materialise_decoder_fwd",
     "lthc_cast_many",
     "lthc_swiglu",
+    "lthc_swiglu_bwd",
     "lthc_gate_add_norm_modulate_fwd",
     "lthc_gate_add_norm_modulate_bwd_workspace_bytes",
     "lthc_gate_add_norm_modulate_bwd",
@@ -129,6 +130,7 @@ def load() -> ctypes.CDLL:
         ],  # fmt: skip
         "lthc_cast_many": [vp, vp, i64, vp, ci, vp],
         "lthc_swiglu": [vp, ci, vp, i64, i64, vp],
+        "lthc_swiglu_bwd": [vp, vp, ci, vp, i64, i64, vp],
         "lthc_gate_add_norm_modulate_bwd": [
             vp, vp, vp, vp, vp, ci, vp, ci, vp, i64, vp, vp, vp, vp, vp, vp, ci, i64, i64, i64, ctypes.c_float, vp, sz,
             vp,

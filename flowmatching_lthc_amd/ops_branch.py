@@ -297,12 +297,38 @@ def _(x):
     return x.new_empty((*x.shape[:-1], x.shape[-1] // 2))
 
 
+@torch.library.custom_op("jit_thc::swiglu_backward", mutates_args=())
+def swiglu_backward(grad: Tensor, x: Tensor) -> Tensor:
+    """Gradient of swiglu for x [..., 2F] and the output gradient [..., F], with eager autograd's roundings."""
+    _on_gpu(x, grad)
+    two_f = x.shape[-1]
+    if two_f % 16 != 0 or tuple(grad.shape) != (*x.shape[:-1], two_f // 2):
+        raise ValueError(f"x [..., 2F] with F % 8 == 0 and grad [..., F] expected, got {tuple(x.shape)}, {tuple(grad.shape)}")
+    x, grad = _aligned(x), _aligned(grad.to(x.dtype))
+    gx = torch.empty_like(x)
+    with _on_device(x):
+        rc = _abi.load().lthc_swiglu_bwd(
+            x.data_ptr(), grad.data_ptr(), _abi.code(x), gx.data_ptr(), x.numel() // two_f if two_f else 0, two_f // 2,
+            _abi.stream_of(x),
+        )  # fmt: skip
+    _abi.check(rc, "lthc_swiglu_bwd")
+    return gx
+
+
+@_fake(swiglu_backward)
+def _(grad, x):
+    return torch.empty_like(x)
+
+
 def _setup_swiglu_ctx(ctx, inputs, output):
     ctx.save_for_backward(inputs[0])
 
 
 def _backward_swiglu(ctx, grad):
     (x,) = ctx.saved_tensors
+    if not _batched(grad):
+        with torch.no_grad():
+            return swiglu_backward(grad, x)
     with torch.enable_grad():
         xl = x.detach().requires_grad_()
         (gx,) = torch.autograd.grad(swiglu_eager(xl), (xl,), (grad,))

@@ -419,6 +419,13 @@ int lthc_cast_many(const void* entries, const void* block_map, int64_t nblocks, 
 int lthc_swiglu(const void* x, int x_dtype, void* out, int64_t rows, int64_t F, void* stream);
 
 /*
+ * BACKWARD of lthc_swiglu: grad [rows, F] -> gx [rows, 2F], both x_dtype, with
+ * the roundings eager autograd of local_thc.py:267-269 makes.  Alignment as
+ * the forward.
+ */
+int lthc_swiglu_bwd(const void* x, const void* grad, int x_dtype, void* gx, int64_t rows, int64_t F, void* stream);
+
+/*
  * GATED RESIDUALS OF THE BRANCH (no reference op: WorkspaceSharedAdaLNBranch.forward,
  * local_thc.py:319-323, evaluates them as eager multiplies and adds).  For
  * tokens t = b*N + n of [B, N, C] tensors and per-sample [B, C] gates:

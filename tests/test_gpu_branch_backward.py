@@ -131,3 +131,24 @@ def test_gate_residual_backward_past_2048_channels():
     gate = torch.randn((2, 2056), generator=gen).to(DEV, torch.bfloat16)
     ours, eager = grads_of(OB.gate_residual, (d, gate, m), (g,)), grads_of(OB.gate_residual_eager, (d, gate, m), (g,))
     check_grads(("d", "gate", "m"), ours, eager, grads_of(OB.gate_residual_eager, (d, gate, m), (g,), torch.float64), torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows,F", [(1, 8), (3, 24), (257, 2056)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_swiglu_backward_bits(rows, F, dtype):
+    print(f"case swiglu backward rows={rows} F={F} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(F)
+    x = (torch.randn((rows, 2 * F), generator=gen) * 3).to(DEV, dtype)
+    special = torch.tensor([0.0, -0.0, 88.0, -88.0, 100.0, -100.0, float("inf"), float("nan")], device=DEV, dtype=dtype)
+    x[0, :8] = special
+    g = torch.randn((rows, F), generator=gen).to(DEV, dtype)
+    (ours,), (eager,) = grads_of(OB.swiglu, (x,), (g,)), grads_of(OB.swiglu_eager, (x,), (g,))
+    assert torch.equal(ours.isnan(), eager.isnan())
+    a, e = ours.nan_to_num().float(), eager.nan_to_num().float()
+    if dtype == torch.float16:
+        # the kernel rounds the gate's gradient to fp32 and then to fp16; torch's own fp16 kernel may fold its last
+        # product and the narrowing into one rounding, so a value next to a tie can differ by one unit: |d| <= 2^-10 |e|
+        # (2^-24 below the normal range), in at most 1 of 1000
+        assert ((a - e).abs() <= 2.0**-10 * e.abs() + 2.0**-24).all() and (a != e).float().mean().item() <= 1e-3
+    else:
+        assert torch.equal(a, e)
