@@ -49,6 +49,8 @@ EXPORTS = (
     "lthc_norm_modulate_bwd_workspace_bytes",
     "lthc_norm_modulate_bwd",
     "lthc_qk_norm_rope",
+    "lthc_qk_norm_rope_bwd_workspace_bytes",
+    "lthc_qk_norm_rope_bwd",
     "lthc_qk_norm_rope_attention",
     "lthc_qk_norm_rope_attention_bwd_workspace_bytes",
     "lthc_qk_norm_rope_attention_bwd",
@@ -136,6 +138,9 @@ def load() -> ctypes.CDLL:
             vp,
         ],  # fmt: skip
         "lthc_gate_residual_bwd": [vp, vp, vp, i64, ci, vp, vp, i64, i64, i64, vp, sz, vp],
+        "lthc_qk_norm_rope_bwd": [
+            vp, vp, vp, ci, vp, vp, ci, vp, vp, ci, vp, vp, ci, i64, i64, i64, i64, ctypes.c_float, vp, sz, vp,
+        ],  # fmt: skip
         "lthc_gate_add_norm_modulate_fwd": [
             vp, vp, vp, ci, vp, ci, vp, vp, i64, vp, vp, vp, i64, i64, i64, ctypes.c_float, vp,
         ],  # fmt: skip
@@ -173,7 +178,7 @@ def load() -> ctypes.CDLL:
     lib.lthc_ws_accumulate_bwd_workspace_bytes.restype = sz
     lib.lthc_norm_modulate_bwd_workspace_bytes.argtypes = [i64, i64, i64]
     lib.lthc_norm_modulate_bwd_workspace_bytes.restype = sz
-    for name in ("lthc_qk_norm_rope_attention_bwd",):
+    for name in ("lthc_qk_norm_rope_attention_bwd", "lthc_qk_norm_rope_bwd"):
         fn = getattr(lib, name + "_workspace_bytes")
         fn.argtypes = [i64, i64, i64, i64]
         fn.restype = sz

@@ -141,9 +141,47 @@ def _setup_qk_ctx(ctx, inputs, output):
     ctx.eps = eps
 
 
+@torch.library.custom_op("jit_thc::qk_norm_rope_backward", mutates_args=())
+def qk_norm_rope_backward(
+    grad_q: Tensor, grad_k: Tensor, qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos: Tensor, sin: Tensor, eps: float
+) -> tuple[Tensor, Tensor]:
+    """(gradient of qkv in qkv's dtype, zero for v, and the fp32 [2, 64] gradients of the q and k norm weights) of
+    qk_norm_rope, with eager autograd's roundings, one pass."""
+    _on_gpu(qkv, grad_q, grad_k, q_weight, k_weight, cos, sin)
+    b, n, h = _check_qk(qkv, q_weight, k_weight, cos, sin)
+    for name, t in (("grad_q", grad_q), ("grad_k", grad_k)):
+        if tuple(t.shape) != (b, n, h, QK_HEAD_DIM):
+            raise ValueError(f"{name} must be [{b},{n},{h},{QK_HEAD_DIM}], got {tuple(t.shape)}")
+    qkv, grad_q, grad_k = _aligned(qkv), _aligned(grad_q.to(qkv.dtype)), _aligned(grad_k.to(qkv.dtype))
+    qw, kw, c, s = _qk_operands(qkv, q_weight, k_weight, cos, sin)
+    dqkv = torch.empty_like(qkv)
+    dw = torch.empty((2, QK_HEAD_DIM), device=qkv.device, dtype=torch.float32)
+    lib = _abi.load()
+    ws = _workspace(lib.lthc_qk_norm_rope_bwd_workspace_bytes(b, n, h, QK_HEAD_DIM), qkv)
+    with _on_device(qkv):
+        rc = lib.lthc_qk_norm_rope_bwd(
+            qkv.data_ptr(), grad_q.data_ptr(), grad_k.data_ptr(), _abi.code(qkv), qw.data_ptr(), kw.data_ptr(),
+            _abi.code(qw), c.data_ptr(), s.data_ptr(), _abi.code(c), dqkv.data_ptr(), dw.data_ptr(), _abi.F32, b, n, h,
+            QK_HEAD_DIM, eps, ws.data_ptr(), ws.numel(), _abi.stream_of(qkv),
+        )  # fmt: skip
+    _abi.check(rc, "lthc_qk_norm_rope_bwd")
+    return dqkv, dw
+
+
+@_fake(qk_norm_rope_backward)
+def _(grad_q, grad_k, qkv, q_weight, k_weight, cos, sin, eps):
+    return torch.empty_like(qkv), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
+
+
 def _backward_qk(ctx, grad_q, grad_k):
     qkv, q_weight, k_weight, cos, sin = ctx.saved_tensors
     need = ctx.needs_input_grad
+    if grad_q is not None and grad_k is not None and not _batched(grad_q, grad_k):
+        with torch.no_grad():
+            dqkv, dw = qk_norm_rope_backward(grad_q, grad_k, qkv, q_weight, k_weight, cos, sin, ctx.eps)
+            dq = dw[0].to(q_weight.dtype) if need[1] else None
+            dk = dw[1].to(k_weight.dtype) if need[2] else None
+        return dqkv if need[0] else None, dq, dk, None, None, None
     with torch.enable_grad():
         leaves = [t.detach().requires_grad_(bool(r)) for t, r in zip((qkv, q_weight, k_weight), need[:3])]
         q, k = qk_norm_rope_eager(leaves[0], leaves[1], leaves[2], cos, sin, ctx.eps)

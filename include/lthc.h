@@ -314,6 +314,18 @@ int lthc_qk_norm_rope(const void* qkv, int x_dtype, const void* q_weight, const 
                       int64_t N, int64_t H, int64_t D, float eps, void* stream);
 
 /*
+ * BACKWARD of lthc_qk_norm_rope: grad_q, grad_k [B, N, H, D] -> dqkv
+ * [B, N, 3, H, D] (x_dtype; v's part zero) and dweights [2, D] (q, k;
+ * dw_dtype), with the roundings eager autograd makes between its ops and
+ * fixed-order fp32 sums.  Shapes, dtypes and alignment as the forward.
+ */
+size_t lthc_qk_norm_rope_bwd_workspace_bytes(int64_t B, int64_t N, int64_t H, int64_t D);
+int lthc_qk_norm_rope_bwd(const void* qkv, const void* grad_q, const void* grad_k, int x_dtype, const void* q_weight,
+                          const void* k_weight, int w_dtype, const void* cos_table, const void* sin_table,
+                          int table_dtype, void* dqkv, void* dweights, int dw_dtype, int64_t B, int64_t N, int64_t H,
+                          int64_t D, float eps, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Q/K RMSNORM + ROPE FUSED WITH THE ATTENTION (no reference op: the reference
  * evaluates WorkspaceAttention.forward, local_thc.py:246-251, as the q/k
  * norms, RoPE and F.scaled_dot_product_attention).  For qkv [B, N, 3, H, D]:

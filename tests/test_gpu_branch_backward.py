@@ -152,3 +152,30 @@ def test_swiglu_backward_bits(rows, F, dtype):
         assert ((a - e).abs() <= 2.0**-10 * e.abs() + 2.0**-24).all() and (a != e).float().mean().item() <= 1e-3
     else:
         assert torch.equal(a, e)
+
+
+# vectors: fewer than one block's 32, an odd number, more than the grid takes in one step (B * N * H > 4 CUs x 256)
+@pytest.mark.parametrize("B,N,H", [(1, 4, 1), (3, 100, 3), (40, 144, 7)])
+@pytest.mark.parametrize("dtype,tdt,wdt", [
+    (torch.float32, torch.float32, torch.float32),
+    (torch.bfloat16, torch.float32, torch.bfloat16),
+    (torch.float16, torch.float16, torch.float32),
+])  # fmt: skip
+def test_qk_norm_rope_backward(B, N, H, dtype, tdt, wdt):
+    print(f"case qk norm rope backward B={B} N={N} H={H} {dtype} {tdt} {wdt}", flush=True)
+    gen = torch.Generator().manual_seed(N)
+    qkv = (torch.randn((B, N, 3, H, 64), generator=gen) * 2).to(DEV, dtype)
+    w0, w1 = ((torch.randn(64, generator=gen) * 0.2 + 1).to(DEV, wdt) for _ in range(2))
+    th = torch.rand((N, 64), generator=gen) * 6.2831853
+    cos, sin = th.cos().to(DEV, tdt), th.sin().to(DEV, tdt)
+    gq, gk = (torch.randn((B, N, H, 64), generator=gen).to(DEV, dtype) for _ in range(2))
+    c, s = cos.to(dtype).double(), sin.to(dtype).double()
+
+    def exact(x, a, b):
+        return qk_exact(x[:, :, 0], a, c, s), qk_exact(x[:, :, 1], b, c, s)
+
+    tensors = (qkv, w0, w1)
+    ours = grads_of(lambda *t: OB.qk_norm_rope(*t, cos, sin, 1e-6), tensors, (gq, gk))
+    eager = grads_of(lambda *t: OB.qk_norm_rope_eager(*t, cos, sin, 1e-6), tensors, (gq, gk))
+    check_grads(("qkv", "q weight", "k weight"), ours, eager, grads_of(exact, tensors, (gq, gk), torch.float64), dtype)
+    assert ours[0][:, :, 2].abs().max().item() == 0.0
