@@ -14,7 +14,7 @@ from typing import Sequence
 
 import torch
 
-from ._build import LIB_PATH
+from ._build import LIB_PATH, OPS_PATH
 
 F32, BF16, F16 = 0, 1, 2
 OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_HIP = 0, 1, 2, 3
@@ -188,6 +188,18 @@ def load() -> ctypes.CDLL:
         fn.restype = sz
     _lib = lib
     return lib
+
+
+def load_torch_ops(missing_ok: bool = False) -> None:
+    """Load the native jit_thc operators (csrc/torch_ops.cpp, linked to the library above) into torch's dispatcher."""
+    if not os.path.exists(OPS_PATH):
+        if missing_ok:
+            return
+        raise RuntimeError(
+            f"{OPS_PATH} is missing: the native LTHC operators must be built "
+            "(python -m flowmatching_lthc_amd._build); there is no fallback"
+        )
+    torch.ops.load_library(OPS_PATH)
 
 
 def check(rc: int, what: str) -> None:

@@ -17,6 +17,11 @@ Every op:
     captured in a HIP graph or traced by ``torch.compile`` (``register_fake``);
   * accumulates in fp32 and rounds once to the output dtype.
 
+The GPU kernels and autograd formulas of the ops the models and the interface
+run are native (``csrc/torch_ops.cpp``, loaded below); their Python bodies here
+carry the schema and refuse other devices.  The remaining ops call the C ABI
+from Python.
+
 Naming follows the reference: the legacy "write" op is the algorithmic READ
 (high-res -> workspace) and the legacy "read" op is the algorithmic WRITE.
 """
@@ -32,6 +37,8 @@ import torch
 from torch import Tensor
 
 from . import _abi
+
+_abi.load_torch_ops(missing_ok=True)  # the GPU kernels and autograd of the ops whose bodies below are _refuse
 
 S = 4  # cell side (taps K = 16)
 K = S * S
@@ -65,7 +72,9 @@ def _register_inductor_fallbacks() -> None:
             continue
         for overload in packet.overloads():
             op = getattr(packet, overload)
-            if op not in lowerings:
+            # composite ops (the two that only open an autograd node) decompose into registered ones
+            composite = torch._C._dispatch_has_kernel_for_dispatch_key(op.name(), "CompositeImplicitAutograd")
+            if op not in lowerings and not composite:
                 make_fallback(op, layout_constraint=tag_to_layout_constraint(get_layout_constraint_tag(op, with_default=True)))
 
 
@@ -98,6 +107,14 @@ def _on_gpu(*ts: Tensor) -> None:
     for t in ts[1:]:
         if t.device != dev:
             raise ValueError(f"all tensors must be on {dev}, got one on {t.device}")
+
+
+def _refuse(t: Tensor):
+    """The Python body of an op whose GPU kernel is native (csrc/torch_ops.cpp): it runs for tensors of other devices
+    only, or where the native operators have not been built."""
+    _on_gpu(t)
+    _abi.load_torch_ops()
+    raise RuntimeError("the native LTHC operators were built after this process imported the package: start it again")
 
 
 def _prep(t: Tensor) -> Tensor:
@@ -172,14 +189,6 @@ def _same_dtype(ref: Tensor, others: Sequence[Tensor]) -> list[Tensor]:
 # ---------------------------------------------------------------------------
 # launches (inputs already checked and prepared)
 # ---------------------------------------------------------------------------
-def _launch_read(x: Tensor, w: Tensor, z: Tensor, b: int, g: int, c: int) -> None:
-    with _on_device(x):
-        rc = _abi.load().lthc_read_fwd(
-            x.data_ptr(), _abi.code(x), w.data_ptr(), _abi.code(w), z.data_ptr(), b, g, S, c, _abi.stream_of(x)
-        )
-    _abi.check(rc, "lthc_read_fwd")
-
-
 def _launch_materialise(base: Tensor | None, dzs: Sequence[Tensor], betas: Sequence[Tensor], out: Tensor) -> None:
     b, g, c = _lo_geom(dzs[0], "dz")
     wd = _abi.code(betas[0])
@@ -216,43 +225,11 @@ def _launch_weight_grad(high: Tensor, lows: Sequence[Tensor]) -> Tensor:
     return out
 
 
-def _launch_materialise_bwd(gr: Tensor, dzs: Sequence[Tensor], betas: Sequence[Tensor], outs: Sequence[Tensor]) -> Tensor:
-    """gdZ_l into outs and the fp32 [L,C,16] gbeta from one pass over gr (lthc_materialise_bwd)."""
-    b, g, c = _hi_geom(gr, "grad_out")
-    L = len(dzs)
-    gb = torch.empty((L, c, K), device=gr.device, dtype=torch.float32)
-    nbytes = _abi.materialise_bwd_workspace_bytes(b, g, S, c, L)
-    ws = torch.empty((max(nbytes, 16),), device=gr.device, dtype=torch.uint8)
-    with _on_device(gr):
-        rc = _abi.load().lthc_materialise_bwd(
-            gr.data_ptr(), _abi.code(gr), _abi.ptr_array(dzs), _abi.ptr_array(betas), _abi.code(betas[0]),
-            _abi.ptr_array(outs), gb.data_ptr(), b, g, S, c, L, ws.data_ptr(), ws.numel(), _abi.stream_of(gr),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_materialise_bwd")
-    return gb
-
-
 @torch.library.custom_op("jit_thc::final_accumulate_backward", mutates_args=())
 def final_accumulate_backward(grad_out: Tensor, dzs: list[Tensor], betas: list[Tensor]) -> tuple[Tensor, Tensor]:
     """(gdZ stack [L,B,M,C] in grad_out.dtype, fp32 [L,C,16] gbeta) of X_L = x0 + sum_l P_l(dz_l): the results of
     the two reference backward ops (_grad_dz_ptr, _grad_beta_ptr) from one pass over grad_out."""
-    _on_gpu(grad_out, *dzs, *betas)
-    b, g, c = _hi_geom(grad_out, "grad_out")
-    L = len(dzs)
-    if L != len(betas) or not 1 <= L <= _abi.MAX_LAYERS:
-        raise ValueError(f"expected 1..{_abi.MAX_LAYERS} dz and as many beta tensors, got {len(dzs)} and {len(betas)}")
-    for i, (dz, bt) in enumerate(zip(dzs, betas)):
-        if tuple(dz.shape) != (b, g * g, c):
-            raise ValueError(f"dz[{i}] must be [{b},{g * g},{c}], got {tuple(dz.shape)}")
-        _check_weight(bt, c, f"beta[{i}]")
-    grad_out = _prep(grad_out)
-    dzs = _same_dtype(grad_out, [_prep(d) for d in dzs])
-    betas = [_prep_w(bt, grad_out.dtype) for bt in betas]
-    if len({bt.dtype for bt in betas}) != 1:
-        betas = [_prep_w(bt.float(), grad_out.dtype) for bt in betas]
-    gdz = torch.empty((L, b, g * g, c), device=grad_out.device, dtype=grad_out.dtype)
-    gb = _launch_materialise_bwd(grad_out, dzs, betas, list(gdz.unbind(0)))
-    return gdz, gb
+    _refuse(grad_out)
 
 
 @_fake(final_accumulate_backward)
@@ -267,14 +244,7 @@ def _(grad_out: Tensor, dzs: list[Tensor], betas: list[Tensor]):
 @torch.library.custom_op("jit_thc::local_write_traceable", mutates_args=())
 def local_write_traceable(x: Tensor, weight: Tensor) -> Tensor:
     """Z[b,m,c] = sum_k weight[c,k] X[b,m,k,c]: x [B,H,H,C] -> z [B,(H/4)^2,C] in x.dtype."""
-    _on_gpu(x, weight)
-    b, g, c = _hi_geom(x)
-    _check_weight(weight, c, "weight")
-    x = _prep(x)
-    w = _prep_w(weight, x.dtype)
-    z = torch.empty((b, g * g, c), device=x.device, dtype=x.dtype)
-    _launch_read(x, w, z, b, g, c)
-    return z
+    _refuse(x)
 
 
 @_fake(local_write_traceable)
@@ -289,14 +259,7 @@ def _(x: Tensor, weight: Tensor) -> Tensor:
 @torch.library.custom_op("jit_thc::local_read_traceable", mutates_args=())
 def local_read_traceable(z: Tensor, weight: Tensor) -> Tensor:
     """X[b,m,k,c] = weight[c,k] Z[b,m,c]: z [B,M,C] -> x [B,4*sqrt(M),4*sqrt(M),C] in z.dtype."""
-    _on_gpu(z, weight)
-    b, g, c = _lo_geom(z)
-    _check_weight(weight, c, "weight")
-    z = _prep(z)
-    w = _prep_w(weight, z.dtype)
-    out = torch.empty((b, g * S, g * S, c), device=z.device, dtype=z.dtype)
-    _launch_materialise(None, [z], [w], out)
-    return out
+    _refuse(z)
 
 
 @_fake(local_read_traceable)
@@ -311,14 +274,7 @@ def _(z: Tensor, weight: Tensor) -> Tensor:
 @torch.library.custom_op("jit_thc::local_weight_grad_traceable", mutates_args=())
 def local_weight_grad_traceable(high: Tensor, low: Tensor) -> Tensor:
     """gW[c,k] = sum_{b,m} high[b,m,k,c] low[b,m,c] in fp32 [C,16] (deterministic order)."""
-    _on_gpu(high, low)
-    b, g, c = _hi_geom(high, "high")
-    bl, gl, cl = _lo_geom(low, "low")
-    if (bl, gl, cl) != (b, g, c):
-        raise ValueError(f"high {tuple(high.shape)} and low {tuple(low.shape)} do not match")
-    high = _prep(high)
-    (low,) = _same_dtype(high, [_prep(low)])
-    return _launch_weight_grad(high, [low])[0]
+    _refuse(high)
 
 
 @_fake(local_weight_grad_traceable)
@@ -327,75 +283,18 @@ def _(high: Tensor, low: Tensor) -> Tensor:
     return high.new_empty((c, K), dtype=torch.float32)
 
 
-def _setup_write_ctx(ctx, inputs, output):
-    x, weight = inputs
-    ctx.save_for_backward(x, weight)
-
-
-def _backward_write(ctx, grad_z):
-    # local_thc_triton_kernels.py:2726-2729
-    x, weight = ctx.saved_tensors
-    grad_x = local_read_traceable(grad_z, weight) if ctx.needs_input_grad[0] else None
-    grad_w = local_weight_grad_traceable(x, grad_z).to(dtype=weight.dtype) if ctx.needs_input_grad[1] else None
-    return grad_x, grad_w
-
-
-def _setup_read_ctx(ctx, inputs, output):
-    z, weight = inputs
-    ctx.save_for_backward(z, weight)
-
-
-def _backward_read(ctx, grad_x):
-    # local_thc_triton_kernels.py:2737-2741
-    z, weight = ctx.saved_tensors
-    grad_z = local_write_traceable(grad_x, weight) if ctx.needs_input_grad[0] else None
-    grad_w = local_weight_grad_traceable(grad_x, z).to(dtype=weight.dtype) if ctx.needs_input_grad[1] else None
-    return grad_z, grad_w
-
-
-torch.library.register_autograd(local_write_traceable, _backward_write, setup_context=_setup_write_ctx)
-torch.library.register_autograd(local_read_traceable, _backward_read, setup_context=_setup_read_ctx)
-
-
 # ---------------------------------------------------------------------------
 # WRITE-ADD  (jit_thc::local_read_add_traceable, local_thc_triton_kernels.py:2713-2723)
 # ---------------------------------------------------------------------------
 @torch.library.custom_op("jit_thc::local_read_add_traceable", mutates_args=())
 def local_read_add_traceable(z: Tensor, weight: Tensor, x: Tensor) -> Tensor:
     """x[b,m,k,c] + weight[c,k] z[b,m,c] in x.dtype, one pass over x (the materialisation with L = 1)."""
-    _on_gpu(z, weight, x)
-    b, g, c = _lo_geom(z)
-    bx, gx, cx = _hi_geom(x)
-    if (bx, gx, cx) != (b, g, c):
-        raise ValueError(f"z {tuple(z.shape)} and x {tuple(x.shape)} do not describe the same cells")
-    _check_weight(weight, c, "weight")
-    x = _prep(x)
-    (z,) = _same_dtype(x, [_prep(z)])
-    w = _prep_w(weight, x.dtype)
-    out = torch.empty_like(x)
-    _launch_materialise(x, [z], [w], out)
-    return out
+    _refuse(z)
 
 
 @_fake(local_read_add_traceable)
 def _(z: Tensor, weight: Tensor, x: Tensor) -> Tensor:
     return torch.empty_like(x)
-
-
-def _setup_read_add_ctx(ctx, inputs, output):
-    z, weight, _ = inputs
-    ctx.save_for_backward(z, weight)
-
-
-def _backward_read_add(ctx, grad_out):
-    # local_thc_triton_kernels.py:2749-2754
-    z, weight = ctx.saved_tensors
-    grad_z = local_write_traceable(grad_out, weight) if ctx.needs_input_grad[0] else None
-    grad_w = local_weight_grad_traceable(grad_out, z).to(dtype=weight.dtype) if ctx.needs_input_grad[1] else None
-    return grad_z, grad_w, grad_out
-
-
-torch.library.register_autograd(local_read_add_traceable, _backward_read_add, setup_context=_setup_read_add_ctx)
 
 
 # ---------------------------------------------------------------------------
@@ -457,7 +356,8 @@ def local_read_add_no_weight_grad(z: Tensor, weight: Tensor, x: Tensor) -> Tenso
 
 
 class _OpenInterface(torch.autograd.Function):
-    """(x, Z0 = R(x)) as one autograd node.
+    """(x, Z0 = R(x)) as one autograd node, for torch.compile's tracing (eager calls open the same node natively:
+    OpenFn, csrc/torch_ops.cpp).
 
     In the lazy forward x feeds both the read and the final materialisation,
     so autograd would write R^T(gZ0) as a full high-res tensor and then add
@@ -496,7 +396,9 @@ def read_with_residual(x: Tensor, weight: Tensor) -> tuple[Tensor, Tensor]:
     Values are those of the two separate uses; the backward of x is
     g_x + R^T(gZ) in one pass instead of autograd's separate write and add.
     """
-    return _OpenInterface.apply(x, weight)
+    if torch.compiler.is_compiling():
+        return _OpenInterface.apply(x, weight)
+    return torch.ops.jit_thc.read_with_residual(x, weight)
 
 
 # ---------------------------------------------------------------------------
@@ -612,16 +514,7 @@ def _check_list(x0: Tensor, dzs: Sequence[Tensor], betas: Sequence[Tensor]) -> i
 @torch.library.custom_op("jit_thc::final_accumulate_list", mutates_args=())
 def final_accumulate_list(x0: Tensor, dzs: list[Tensor], betas: list[Tensor]) -> Tensor:
     """X_L = x0 + sum_l betas[l][c,k] dzs[l][b,m,c] in x0.dtype, one pass, the L layers passed as lists."""
-    _on_gpu(x0, *dzs, *betas)
-    _check_list(x0, dzs, betas)
-    x0 = _prep(x0)
-    dzs = _same_dtype(x0, [_prep(d) for d in dzs])
-    betas = [_prep_w(bt, x0.dtype) for bt in betas]
-    if len({bt.dtype for bt in betas}) != 1:
-        betas = [bt.float() for bt in betas]
-    out = torch.empty_like(x0)
-    _launch_materialise(x0, dzs, betas, out)
-    return out
+    _refuse(x0)
 
 
 @_fake(final_accumulate_list)
@@ -669,45 +562,10 @@ def _(grad_out: Tensor, dzs: list[Tensor]) -> Tensor:
     return grad_out.new_empty((len(dzs), grad_out.shape[3], K), dtype=torch.float32)
 
 
-def _setup_final_accumulate_list_ctx(ctx, inputs, output):
-    _, dzs, betas = inputs
-    ctx.save_for_backward(*dzs, *betas)
-    ctx.L = len(dzs)
-
-
-def _backward_final_accumulate_list(ctx, grad_out):
-    saved = ctx.saved_tensors
-    dzs, betas = saved[: ctx.L], saved[ctx.L :]
-    grad_out = grad_out.contiguous()
-    if ctx.needs_input_grad[1] and ctx.needs_input_grad[2]:  # both from one pass over grad_out
-        gdz, gb = final_accumulate_backward(grad_out, list(dzs), list(betas))
-        return grad_out, list(gdz.unbind(0)), [g.to(dtype=bt.dtype) for g, bt in zip(gb.unbind(0), betas, strict=True)]
-    grad_dzs = final_accumulate_list_grad_dz(grad_out, list(betas)) if ctx.needs_input_grad[1] else None
-    grad_betas = None
-    if ctx.needs_input_grad[2]:
-        gb = final_accumulate_list_grad_beta(grad_out, list(dzs))
-        grad_betas = [g.to(dtype=bt.dtype) for g, bt in zip(gb.unbind(0), betas, strict=True)]
-    return grad_out, grad_dzs, grad_betas
-
-
-torch.library.register_autograd(
-    final_accumulate_list, _backward_final_accumulate_list, setup_context=_setup_final_accumulate_list_ctx
-)
-
-
 # ---------------------------------------------------------------------------
 # MATERIALISE, 12 separate layers (jit_thc::final_accumulate_b4_12_traceable,
 # local_thc_triton_kernels.py:1669-1736) and its backward ops (:1800-1919)
 # ---------------------------------------------------------------------------
-def _check_12(x0: Tensor, dzs: Sequence[Tensor], betas: Sequence[Tensor]) -> None:
-    b, g, c = _hi_geom(x0, "x0")
-    for i, dz in enumerate(dzs):
-        if tuple(dz.shape) != (b, g * g, c):
-            raise ValueError(f"dz{i} must be [{b},{g * g},{c}], got {tuple(dz.shape)}")
-    for i, bt in enumerate(betas):
-        _check_weight(bt, c, f"beta{i}")
-
-
 @torch.library.custom_op("jit_thc::final_accumulate_b4_12_traceable", mutates_args=())
 def final_accumulate_b4_12_traceable(
     x0: Tensor,
@@ -717,18 +575,7 @@ def final_accumulate_b4_12_traceable(
     beta6: Tensor, beta7: Tensor, beta8: Tensor, beta9: Tensor, beta10: Tensor, beta11: Tensor,
 ) -> Tensor:  # fmt: skip
     """X_L = x0 + sum_{l<12} beta_l[c,k] dz_l[b,m,c]; one pass over X0, stored once in x0.dtype."""
-    dzs = [dz0, dz1, dz2, dz3, dz4, dz5, dz6, dz7, dz8, dz9, dz10, dz11]
-    betas = [beta0, beta1, beta2, beta3, beta4, beta5, beta6, beta7, beta8, beta9, beta10, beta11]
-    _on_gpu(x0, *dzs, *betas)
-    _check_12(x0, dzs, betas)
-    x0 = _prep(x0)
-    dzs = _same_dtype(x0, [_prep(d) for d in dzs])
-    betas = [_prep_w(bt, x0.dtype) for bt in betas]
-    if len({bt.dtype for bt in betas}) != 1:
-        betas = [_prep_w(bt.float(), x0.dtype) for bt in betas]
-    out = torch.empty_like(x0)
-    _launch_materialise(x0, dzs, betas, out)
-    return out
+    _refuse(x0)
 
 
 @_fake(final_accumulate_b4_12_traceable)
@@ -786,65 +633,13 @@ def _(grad_out, *dzs):
     return grad_out.new_empty((12, grad_out.shape[3], K), dtype=torch.float32)
 
 
-def _setup_final_accumulate_12_ctx(ctx, inputs, output):
-    ctx.save_for_backward(*inputs[1:])
-
-
-def _backward_final_accumulate_12(ctx, grad_out):
-    # local_thc_triton_kernels.py:1901-1912: grad_x0 is grad_out itself.
-    saved = ctx.saved_tensors
-    dzs, betas = saved[:12], saved[12:]
-    grad_out = grad_out.contiguous()
-    need = ctx.needs_input_grad
-    grad_dzs = (None,) * 12
-    grad_betas = (None,) * 12
-    if any(need[1:13]) and any(need[13:25]):  # both from one pass over grad_out
-        gdz, gb = final_accumulate_backward(grad_out, list(dzs), list(betas))
-        grad_betas = tuple(g.to(dtype=bt.dtype) for g, bt in zip(gb.unbind(0), betas, strict=True))
-        return (grad_out, *gdz.unbind(0), *grad_betas)
-    if any(need[1:13]):
-        grad_dzs = tuple(final_accumulate_b4_12_grad_dz_ptr_traceable(grad_out, *betas).unbind(0))
-    if any(need[13:25]):
-        gb = final_accumulate_b4_12_grad_beta_ptr_traceable(grad_out, *dzs)
-        grad_betas = tuple(g.to(dtype=bt.dtype) for g, bt in zip(gb.unbind(0), betas, strict=True))
-    return (grad_out, *grad_dzs, *grad_betas)
-
-
-torch.library.register_autograd(
-    final_accumulate_b4_12_traceable, _backward_final_accumulate_12, setup_context=_setup_final_accumulate_12_ctx
-)
-
-
 # ---------------------------------------------------------------------------
 # LAZY WORKSPACE RECURRENCE  (no reference op: local_thc.py:1325-1328 is eager torch)
 # ---------------------------------------------------------------------------
-def _check_recur(z: Tensor, dz: Tensor, gamma: Tensor) -> int:
-    if z.shape != dz.shape or z.dim() < 1:
-        raise ValueError(f"z {tuple(z.shape)} and dz {tuple(dz.shape)} must have the same shape")
-    c = z.shape[-1]
-    if tuple(gamma.shape) != (c,):
-        raise ValueError(f"gamma must be [{c}], got {tuple(gamma.shape)}")
-    if c % 4 != 0:
-        raise ValueError(f"channels {c} must be a multiple of 4")
-    _abi.code(gamma)
-    return c
-
-
 @torch.library.custom_op("jit_thc::lazy_workspace_update", mutates_args=())
 def lazy_workspace_update(z: Tensor, dz: Tensor, gamma: Tensor) -> Tensor:
     """Z_{l+1} = Z_l + gamma[c] * dZ_l computed as fma(gamma, dz, z), in the promoted dtype of z and dz."""
-    _on_gpu(z, dz, gamma)
-    c = _check_recur(z, dz, gamma)
-    dt = torch.promote_types(z.dtype, dz.dtype)
-    z, dz, gamma = _prep(z.to(dt)), _prep(dz.to(dt)), _prep(gamma)
-    out = torch.empty_like(z)
-    with _on_device(z):
-        rc = _abi.load().lthc_recur_fwd(
-            z.data_ptr(), dz.data_ptr(), _abi.code(z), gamma.data_ptr(), _abi.code(gamma), out.data_ptr(),
-            z.numel() // c, c, _abi.stream_of(z),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_recur_fwd")
-    return out
+    _refuse(z)
 
 
 @_fake(lazy_workspace_update)
@@ -857,26 +652,7 @@ def lazy_workspace_update_backward(
     grad: Tensor, dz: Tensor, gamma: Tensor, gdz_add: Tensor | None = None
 ) -> tuple[Tensor, Tensor]:
     """(gamma * grad [+ gdz_add] in grad.dtype, fp32 [C] sum over rows of grad * dz)."""
-    _on_gpu(grad, dz, gamma)
-    c = _check_recur(grad, dz, gamma)
-    grad = _prep(grad)
-    (dz,) = _same_dtype(grad, [_prep(dz)])
-    if gdz_add is not None:
-        if gdz_add.shape != grad.shape:
-            raise ValueError(f"gdz_add {tuple(gdz_add.shape)} must match grad {tuple(grad.shape)}")
-        (gdz_add,) = _same_dtype(grad, [_prep(gdz_add)])
-    gamma = _prep(gamma)
-    rows = grad.numel() // c
-    gdz = torch.empty_like(grad)
-    ggamma = torch.empty((c,), device=grad.device, dtype=torch.float32)
-    ws = torch.empty((max(_abi.recur_bwd_workspace_bytes(rows, c), 16),), device=grad.device, dtype=torch.uint8)
-    with _on_device(grad):
-        rc = _abi.load().lthc_recur_bwd(
-            grad.data_ptr(), dz.data_ptr(), _abi.ptr(gdz_add), _abi.code(grad), gamma.data_ptr(), _abi.code(gamma),
-            gdz.data_ptr(), ggamma.data_ptr(), rows, c, ws.data_ptr(), ws.numel(), _abi.stream_of(grad),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_recur_bwd")
-    return gdz, ggamma
+    _refuse(grad)
 
 
 @_fake(lazy_workspace_update_backward)
@@ -891,30 +667,7 @@ def lazy_workspace_update_backward_sum(
     """(g = grad + grad_branch rounded to grad.dtype, gamma * g [+ gdz_add], [C] sum over rows of g * dz in fp32,
     rounded once to gamma's dtype): lazy_workspace_update_backward of the two gradients of z_next, summed in the
     same pass."""
-    _on_gpu(grad, grad_branch, dz, gamma)
-    c = _check_recur(grad, dz, gamma)
-    if grad_branch.shape != grad.shape:
-        raise ValueError(f"grad_branch {tuple(grad_branch.shape)} must match grad {tuple(grad.shape)}")
-    grad = _prep(grad)
-    dz, grad_branch = _same_dtype(grad, [_prep(dz), _prep(grad_branch)])
-    if gdz_add is not None:
-        if gdz_add.shape != grad.shape:
-            raise ValueError(f"gdz_add {tuple(gdz_add.shape)} must match grad {tuple(grad.shape)}")
-        (gdz_add,) = _same_dtype(grad, [_prep(gdz_add)])
-    gamma = _prep(gamma)
-    rows = grad.numel() // c
-    gsum = torch.empty_like(grad)
-    gdz = torch.empty_like(grad)
-    ggamma = torch.empty((c,), device=grad.device, dtype=gamma.dtype)
-    ws = torch.empty((max(_abi.recur_bwd_workspace_bytes(rows, c), 16),), device=grad.device, dtype=torch.uint8)
-    with _on_device(grad):
-        rc = _abi.load().lthc_recur_bwd_sum(
-            grad.data_ptr(), grad_branch.data_ptr(), dz.data_ptr(), _abi.ptr(gdz_add), _abi.code(grad),
-            gamma.data_ptr(), _abi.code(gamma), gsum.data_ptr(), gdz.data_ptr(), ggamma.data_ptr(), _abi.code(ggamma),
-            rows, c, ws.data_ptr(), ws.numel(), _abi.stream_of(grad),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_recur_bwd_sum")
-    return gsum, gdz, ggamma
+    _refuse(grad)
 
 
 @_fake(lazy_workspace_update_backward_sum)
@@ -922,29 +675,9 @@ def _(grad: Tensor, grad_branch: Tensor, dz: Tensor, gamma: Tensor, gdz_add: Ten
     return torch.empty_like(grad), torch.empty_like(grad), grad.new_empty((grad.shape[-1],), dtype=gamma.dtype)
 
 
-def _setup_recur_ctx(ctx, inputs, output):
-    _, dz, gamma = inputs
-    ctx.save_for_backward(dz, gamma)
-    ctx.z_dtype = inputs[0].dtype
-
-
-def _backward_recur(ctx, grad):
-    dz, gamma = ctx.saved_tensors
-    need = ctx.needs_input_grad
-    grad_z = grad.to(ctx.z_dtype) if need[0] else None
-    grad_dz = grad_gamma = None
-    if need[1] or need[2]:
-        gdz, gg = lazy_workspace_update_backward(grad, dz, gamma)
-        grad_dz = gdz.to(dz.dtype) if need[1] else None
-        grad_gamma = gg.to(gamma.dtype) if need[2] else None
-    return grad_z, grad_dz, grad_gamma
-
-
-torch.library.register_autograd(lazy_workspace_update, _backward_recur, setup_context=_setup_recur_ctx)
-
-
 class _RecurStep(torch.autograd.Function):
-    """(Z_{l+1} = Z_l + gamma * dZ_l, dZ_l) as one autograd node, or (Z_{l+1}, Z_{l+1}', dZ_l) with `split`.
+    """(Z_{l+1} = Z_l + gamma * dZ_l, dZ_l) as one autograd node, or (Z_{l+1}, Z_{l+1}', dZ_l) with `split`; for
+    torch.compile's tracing (eager calls open the same node natively: StepFn, csrc/torch_ops.cpp).
 
     In the lazy forward dZ_l feeds both the recurrence and the final
     materialisation, so autograd would add the two gradients of dZ_l in a
@@ -996,7 +729,9 @@ def lazy_workspace_step(z: Tensor, dz: Tensor, gamma: Tensor, split: bool = Fals
     split=True returns (z_next, z_next for the branch, dz): the same values, with z_next's two
     gradients (next step, branch) summed by that launch too.
     """
-    return _RecurStep.apply(z, dz, gamma, split)
+    if torch.compiler.is_compiling():
+        return _RecurStep.apply(z, dz, gamma, split)
+    return tuple(torch.ops.jit_thc.lazy_workspace_step(z, dz, gamma, split))
 
 
 # ---------------------------------------------------------------------------
@@ -1005,23 +740,7 @@ def lazy_workspace_step(z: Tensor, dz: Tensor, gamma: Tensor, split: bool = Fals
 @torch.library.custom_op("jit_thc::lazy_gamma_stack", mutates_args=())
 def lazy_gamma_stack(alpha: Tensor, beta_stack: Tensor) -> Tensor:
     """fp32 [L,C] of gamma_l = sum_k alpha * beta_l (LayerLocalWrite.gamma_from_alpha for all layers)."""
-    _on_gpu(alpha, beta_stack)
-    if alpha.dim() != 2 or beta_stack.dim() != 3 or tuple(beta_stack.shape[1:]) != tuple(alpha.shape):
-        raise ValueError(f"alpha [C,K] and beta_stack [L,C,K] expected, got {tuple(alpha.shape)}, {tuple(beta_stack.shape)}")
-    L = beta_stack.shape[0]
-    if not 1 <= L <= _abi.MAX_LAYERS:
-        raise ValueError(f"depth {L} outside 1..{_abi.MAX_LAYERS}")
-    (beta_stack,) = _same_dtype(alpha, [beta_stack])
-    alpha, beta_stack = alpha.contiguous(), beta_stack.contiguous()
-    c, k = alpha.shape
-    out = torch.empty((L, c), device=alpha.device, dtype=torch.float32)
-    with _on_device(alpha):
-        rc = _abi.load().lthc_gamma(
-            alpha.data_ptr(), _abi.ptr_array(list(beta_stack.unbind(0))), _abi.code(alpha), out.data_ptr(),
-            _abi.F32, c, k, L, _abi.stream_of(alpha),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_gamma")
-    return out
+    _refuse(alpha)
 
 
 @_fake(lazy_gamma_stack)
@@ -1058,34 +777,12 @@ def lazy_gamma_rounded_eager(alpha: Tensor, betas: Sequence[Tensor], dtype: torc
 def lazy_gamma_rounded(alpha: Tensor, betas: list[Tensor], dtype: torch.dtype) -> Tensor:
     """[L, C] in `dtype` of r(sum_k r(r(alpha) r(beta_l))), r = round to `dtype`, the sum in fp32: the block hooks'
     gamma_from_alpha(shared_read.alpha(dtype)) for all layers in one launch."""
-    _on_gpu(alpha, *betas)
-    if alpha.dim() != 2 or not betas or any(tuple(b.shape) != tuple(alpha.shape) for b in betas):
-        raise ValueError(f"alpha [C,K] and L betas of the same shape expected, got {tuple(alpha.shape)}")
-    if not 1 <= len(betas) <= _abi.MAX_LAYERS:
-        raise ValueError(f"depth {len(betas)} outside 1..{_abi.MAX_LAYERS}")
-    bd = betas[0].dtype
-    betas = [b.contiguous() if b.dtype == bd else b.to(bd).contiguous() for b in betas]
-    alpha = alpha.contiguous()
-    c, k = alpha.shape
-    out = torch.empty((len(betas), c), device=alpha.device, dtype=dtype)
-    with _on_device(alpha):
-        rc = _abi.load().lthc_gamma_rounded(
-            alpha.data_ptr(), _abi.code(alpha), _abi.ptr_array(betas), _abi.code(betas[0]), out.data_ptr(),
-            _abi.code(out), c, k, len(betas), _abi.stream_of(alpha),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_gamma_rounded")
-    return out
+    _refuse(alpha)
 
 
 @_fake(lazy_gamma_rounded)
 def _(alpha: Tensor, betas: list[Tensor], dtype: torch.dtype) -> Tensor:
     return alpha.new_empty((len(betas), alpha.shape[0]), dtype=dtype)
-
-
-def _setup_gamma_rounded_ctx(ctx, inputs, output):
-    alpha, betas, dtype = inputs
-    ctx.save_for_backward(alpha, *betas)
-    ctx.dtype = dtype
 
 
 @torch.library.custom_op("jit_thc::lazy_gamma_rounded_backward", mutates_args=())
@@ -1095,22 +792,7 @@ def lazy_gamma_rounded_backward(
     """Eager autograd's values for lazy_gamma_rounded_eager from one lthc_gamma_rounded_bwd launch: (grad of
     alpha, or an empty tensor when not needed; grads of the betas in the first beta's dtype, or an empty list).
     An op of its own so that the backward is opaque to torch.compile's tracing."""
-    _on_gpu(grad, alpha, *betas)
-    bd = betas[0].dtype
-    betas = [b.contiguous() if b.dtype == bd else b.to(bd).contiguous() for b in betas]
-    alpha = alpha.contiguous()
-    grad = grad.contiguous()
-    ga = torch.empty_like(alpha) if need_alpha else None
-    gbs = [torch.empty_like(b) for b in betas] if need_beta else None
-    c, k = alpha.shape
-    with _on_device(alpha):
-        rc = _abi.load().lthc_gamma_rounded_bwd(
-            grad.data_ptr(), alpha.data_ptr(), _abi.code(alpha), _abi.ptr_array(betas), _abi.code(betas[0]),
-            _abi.ptr(ga), _abi.ptr_array(gbs) if gbs is not None else None, _abi.code(grad), c, k, len(betas),
-            _abi.stream_of(alpha),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_gamma_rounded_bwd")
-    return (ga if ga is not None else alpha.new_empty((0,))), (gbs if gbs is not None else [])
+    _refuse(grad)
 
 
 @_fake(lazy_gamma_rounded_backward)
@@ -1120,41 +802,10 @@ def _(grad: Tensor, alpha: Tensor, betas: list[Tensor], need_alpha: bool, need_b
     return ga, gbs
 
 
-def _backward_gamma_rounded(ctx, grad):
-    """Eager autograd's values for lazy_gamma_rounded_eager, from one lthc_gamma_rounded_bwd launch."""
-    alpha, *betas = ctx.saved_tensors
-    need_a, need_b = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-    if not (need_a or need_b):
-        return None, None, None
-    ga, gbs = lazy_gamma_rounded_backward(grad.to(ctx.dtype), alpha, betas, bool(need_a), bool(need_b))
-    gbs = [g if g.dtype == b.dtype else g.to(b.dtype) for g, b in zip(gbs, betas)] if need_b else None
-    return (ga if need_a else None), gbs, None
-
-
-torch.library.register_autograd(lazy_gamma_rounded, _backward_gamma_rounded, setup_context=_setup_gamma_rounded_ctx)
-
-
 # ---------------------------------------------------------------------------
 # FINAL-LAYER RMSNORM + MODULATE (no reference op: FinalLayerSharedAdaLN's
 # norm_final + modulate, local_thc.py:870-873, is eager torch)
 # ---------------------------------------------------------------------------
-def _check_norm(x: Tensor, weight: Tensor, shift: Tensor, scale: Tensor) -> tuple[int, int, int]:
-    if x.dim() != 3:
-        raise ValueError(f"x must be [B,N,C], got {tuple(x.shape)}")
-    b, n, c = x.shape
-    if tuple(weight.shape) != (c,) or tuple(shift.shape) != (b, c) or tuple(scale.shape) != (b, c):
-        raise ValueError(
-            f"weight [{c}], shift and scale [{b},{c}] expected, got {tuple(weight.shape)}, "
-            f"{tuple(shift.shape)}, {tuple(scale.shape)}"
-        )
-    if shift.dtype != x.dtype or scale.dtype != x.dtype:
-        raise ValueError(f"shift and scale must have x's dtype {x.dtype}, got {shift.dtype}, {scale.dtype}")
-    if c % 4 != 0 or c > 2048:
-        raise ValueError(f"channels {c} must be a multiple of 4 and at most 2048")
-    _abi.code(x)
-    return b, n, c
-
-
 def _mod_rows(*ts: Tensor, elems: int = 4) -> tuple[list[Tensor], int]:
     """Per-sample [B, C] vectors as (tensors, common row stride): strided rows of one buffer (chunks of the shared
     AdaLN vector) are used in place when their rows are contiguous, share a stride that is a multiple of `elems`
@@ -1181,20 +832,7 @@ def _norm_weight(weight: Tensor) -> Tensor:
 @torch.library.custom_op("jit_thc::norm_modulate", mutates_args=())
 def norm_modulate(x: Tensor, weight: Tensor, shift: Tensor, scale: Tensor, eps: float) -> tuple[Tensor, Tensor]:
     """(modulate(RMSNorm(x), shift, scale) in x.dtype, fp32 [B*N] inverse RMS) in one pass over x."""
-    _on_gpu(x, weight, shift, scale)
-    b, n, c = _check_norm(x, weight, shift, scale)
-    x = _prep(x)
-    (shift, scale), ld = _mod_rows(shift, scale)
-    w = _norm_weight(weight)
-    y = torch.empty_like(x)
-    inv = torch.empty((b * n,), device=x.device, dtype=torch.float32)
-    with _on_device(x):
-        rc = _abi.load().lthc_norm_modulate_fwd(
-            x.data_ptr(), _abi.code(x), w.data_ptr(), _abi.code(w), shift.data_ptr(), scale.data_ptr(), ld,
-            y.data_ptr(), inv.data_ptr(), b, n, c, eps, _abi.stream_of(x),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_norm_modulate_fwd")
-    return y, inv
+    _refuse(x)
 
 
 @_fake(norm_modulate)
@@ -1207,25 +845,7 @@ def norm_modulate_backward(
     grad: Tensor, x: Tensor, weight: Tensor, scale: Tensor, inv: Tensor
 ) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """(dx in x.dtype, dweight fp32 [C], dshift fp32 [B,C], dscale fp32 [B,C])."""
-    _on_gpu(grad, x, weight, scale, inv)
-    b, n, c = _check_norm(x, weight, scale, scale)
-    (grad,) = _same_dtype(x, [_prep(grad)])
-    x, inv = _prep(x), inv.float().contiguous()
-    (scale,), ld = _mod_rows(scale)
-    w = _norm_weight(weight)
-    gx = torch.empty_like(x)
-    gw = torch.empty((c,), device=x.device, dtype=torch.float32)
-    gsh = torch.empty((b, c), device=x.device, dtype=torch.float32)
-    gsc = torch.empty((b, c), device=x.device, dtype=torch.float32)
-    ws = torch.empty((max(_abi.norm_modulate_bwd_workspace_bytes(b, n, c), 16),), device=x.device, dtype=torch.uint8)
-    with _on_device(x):
-        rc = _abi.load().lthc_norm_modulate_bwd(
-            grad.data_ptr(), x.data_ptr(), _abi.code(x), w.data_ptr(), _abi.code(w), scale.data_ptr(), ld,
-            inv.data_ptr(), gx.data_ptr(), gw.data_ptr(), gsh.data_ptr(), gsc.data_ptr(), b, n, c, ws.data_ptr(),
-            ws.numel(), _abi.stream_of(x),
-        )  # fmt: skip
-    _abi.check(rc, "lthc_norm_modulate_bwd")
-    return gx, gw, gsh, gsc
+    _refuse(grad)
 
 
 @_fake(norm_modulate_backward)
@@ -1233,22 +853,6 @@ def _(grad: Tensor, x: Tensor, weight: Tensor, scale: Tensor, inv: Tensor):
     b, n, c = x.shape
     f32 = torch.float32
     return torch.empty_like(x), x.new_empty((c,), dtype=f32), x.new_empty((b, c), dtype=f32), x.new_empty((b, c), dtype=f32)
-
-
-def _setup_norm_ctx(ctx, inputs, output):
-    x, weight, shift, scale, _ = inputs
-    ctx.save_for_backward(x, weight, scale, output[1])
-    ctx.dtypes = (weight.dtype, shift.dtype, scale.dtype)
-
-
-def _backward_norm(ctx, grad_y, grad_inv):
-    x, weight, scale, inv = ctx.saved_tensors
-    gx, gw, gsh, gsc = norm_modulate_backward(grad_y.contiguous(), x, weight, scale, inv)
-    wd, shd, scd = ctx.dtypes
-    return gx, gw.to(wd), gsh.to(shd), gsc.to(scd), None
-
-
-torch.library.register_autograd(norm_modulate, _backward_norm, setup_context=_setup_norm_ctx)
 
 
 # ---------------------------------------------------------------------------

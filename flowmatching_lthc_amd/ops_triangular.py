@@ -45,6 +45,7 @@ from .ops import (
     _on_gpu,
     _prep,
     _prep_w,
+    _refuse,
     _same_dtype,
 )
 
@@ -117,8 +118,7 @@ def ws_accumulate_backward(grad: Tensor, dzs: list[Tensor], gamma: Tensor, L: in
     """_ws_backward as an op (the triangular ops' autograd backwards call it, so torch.compile traces them as one
     opaque node): ([gamma[i] * grad for i < L] or [] without want_dz, fp32 [L, C] sum grad * dzs[i] or an empty
     tensor when dzs is empty)."""
-    gdz, gg = _ws_backward(grad, dzs if dzs else None, gamma, L, want_dz)
-    return (gdz if gdz is not None else []), (gg if gg is not None else grad.new_empty((0,), dtype=torch.float32))
+    _refuse(grad)
 
 
 @_fake(ws_accumulate_backward)
@@ -205,7 +205,7 @@ torch.library.register_autograd(triangular_accumulate_traceable, _backward_tri, 
 @torch.library.custom_op("jit_thc::triangular_accumulate_list", mutates_args=())
 def triangular_accumulate_list(base: Tensor, dzs: list[Tensor], gamma: Tensor) -> Tensor:
     """base + sum_{i < len(dzs)} gamma[i][c] * dzs[i] for base [B,M,C], gamma [>= len(dzs), C]."""
-    return _ws_forward(base, dzs, gamma)
+    _refuse(base)
 
 
 @_fake(triangular_accumulate_list)
@@ -213,46 +213,10 @@ def _(base: Tensor, dzs: list[Tensor], gamma: Tensor) -> Tensor:
     return torch.empty_like(base)
 
 
-def _setup_tri_list_ctx(ctx, inputs, output):
-    _, dzs, gamma = inputs
-    ctx.save_for_backward(*dzs, gamma)
-    ctx.L = len(dzs)
-
-
-def _backward_tri_list(ctx, grad_out):
-    saved = ctx.saved_tensors
-    dzs, gamma = list(saved[: ctx.L]), saved[ctx.L]
-    grad_out = grad_out.contiguous()
-    need = ctx.needs_input_grad
-    gdz, gg = _ws_backward_op(grad_out, dzs if need[2] else None, gamma, ctx.L, need[1])
-    grad_gamma = None
-    if gg is not None:
-        if gamma.shape[0] > ctx.L:
-            full = torch.zeros(gamma.shape, device=gg.device, dtype=torch.float32)
-            full[: ctx.L] = gg
-            gg = full
-        grad_gamma = gg.to(gamma.dtype)
-    return grad_out, gdz, grad_gamma
-
-
-torch.library.register_autograd(triangular_accumulate_list, _backward_tri_list, setup_context=_setup_tri_list_ctx)
-
-
 # ---------------------------------------------------------------------------
 # 12 separate layers (:2015-2157) and the active-prefix forms (:2161-2488)
 # ---------------------------------------------------------------------------
 _DZ12 = ", ".join(f"Tensor dz{i}" for i in range(12))
-
-
-def _tri12_forward(base: Tensor, dzs: Sequence[Tensor], gamma: Tensor, active: int) -> Tensor:
-    if base.dim() != 3 or gamma.dim() != 2 or tuple(gamma.shape) != (12, base.shape[2]):
-        raise ValueError(
-            f"triangular_accumulate_b4_12 expects base [B,M,C] and gamma [12,C], got {tuple(base.shape)} and {tuple(gamma.shape)}"
-        )
-    for i, dz in enumerate(dzs):
-        if dz.shape != base.shape:
-            raise ValueError(f"triangular_accumulate_b4_12 dz{i} shape {tuple(dz.shape)} does not match base {tuple(base.shape)}")
-    return _ws_forward(base, list(dzs[:active]), gamma)
 
 
 def _tri12_grad_dz(grad_out: Tensor, gamma: Tensor, active: int) -> Tensor:
@@ -294,11 +258,6 @@ def _check_active(active: int) -> int:
     return int(active)
 
 
-@torch.library.impl("jit_thc::triangular_accumulate_b4_12_ptr_traceable", "CUDA")
-def _tri12_impl(base, *args):
-    return _tri12_forward(base, args[:12], args[12], 12)
-
-
 @torch.library.impl("jit_thc::triangular_accumulate_b4_12_ptr_grad_dz", "CUDA")
 def _tri12_grad_dz_impl(grad_out, gamma):
     return _tri12_grad_dz(grad_out, gamma, 12)
@@ -307,11 +266,6 @@ def _tri12_grad_dz_impl(grad_out, gamma):
 @torch.library.impl("jit_thc::triangular_accumulate_b4_12_ptr_grad_gamma", "CUDA")
 def _tri12_grad_gamma_impl(grad_out, *args):
     return _tri12_grad_gamma(grad_out, args[:12], args[12], 12)
-
-
-@torch.library.impl("jit_thc::triangular_accumulate_b4_12_ptr_active", "CUDA")
-def _tri12a_impl(base, *args):
-    return _tri12_forward(base, args[:12], args[12], _check_active(args[13]))
 
 
 @torch.library.impl("jit_thc::triangular_accumulate_b4_12_ptr_active_grad_dz", "CUDA")
@@ -372,47 +326,6 @@ def _(grad_out, *args):
     return grad_out.new_empty((12, grad_out.shape[-1]), dtype=torch.float32)
 
 
-def _setup_tri12_ctx(ctx, inputs, output):
-    ctx.save_for_backward(*inputs[1:14])
-    ctx.active = int(inputs[14]) if len(inputs) > 14 else 12
-
-
-def _tri12_grads(ctx, grad_out) -> tuple:
-    """Gradients of (base, dz0..dz11, gamma).  local_thc_triton_kernels.py:2141-2151 and :2470-2482:
-    grad_base is grad_out itself; the layers beyond the active prefix get no gradient."""
-    saved = ctx.saved_tensors
-    dzs, gamma, active = saved[:12], saved[12], ctx.active
-    grad_out = grad_out.contiguous()
-    need = ctx.needs_input_grad
-    want_dz = any(need[1 : 1 + active])
-    gdz, gg = _ws_backward_op(grad_out, list(dzs[:active]) if need[13] else None, gamma, active, want_dz)
-    grad_dzs = (tuple(gdz) if gdz is not None else (None,) * active) + (None,) * (12 - active)
-    grad_gamma = None
-    if gg is not None:
-        if active < 12:
-            full = torch.zeros((12, gamma.shape[1]), device=gg.device, dtype=torch.float32)
-            full[:active] = gg
-            gg = full
-        grad_gamma = gg.to(gamma.dtype)
-    return (grad_out, *grad_dzs, grad_gamma)
-
-
-def _backward_tri12(ctx, grad_out):
-    return _tri12_grads(ctx, grad_out)
-
-
-def _backward_tri12_active(ctx, grad_out):
-    return _tri12_grads(ctx, grad_out) + (None,)  # no gradient for the int `active`
-
-
-torch.library.register_autograd(
-    "jit_thc::triangular_accumulate_b4_12_ptr_traceable", _backward_tri12, setup_context=_setup_tri12_ctx
-)
-torch.library.register_autograd(
-    "jit_thc::triangular_accumulate_b4_12_ptr_active", _backward_tri12_active, setup_context=_setup_tri12_ctx
-)
-
-
 def triangular_accumulate_b4_12_ptr_traceable(base, *args):
     return torch.ops.jit_thc.triangular_accumulate_b4_12_ptr_traceable(base, *args)
 
@@ -428,7 +341,6 @@ def _make_active_op(active: int):
     torch.library.define(f"jit_thc::{name}", f"(Tensor base, {_DZ12}, Tensor gamma) -> Tensor")
     torch.library.define(f"jit_thc::{name}_grad_dz", "(Tensor grad_out, Tensor gamma) -> Tensor")
     torch.library.define(f"jit_thc::{name}_grad_gamma", f"(Tensor grad_out, {_DZ12}, Tensor gamma) -> Tensor")
-    torch.library.impl(f"jit_thc::{name}", "CUDA")(lambda base, *a: _tri12_forward(base, a[:12], a[12], active))
     torch.library.impl(f"jit_thc::{name}_grad_dz", "CUDA")(lambda g, gamma: _tri12_grad_dz(g, gamma, active))
     torch.library.impl(f"jit_thc::{name}_grad_gamma", "CUDA")(lambda g, *a: _tri12_grad_gamma(g, a[:12], a[12], active))
     for suffix in ("", "_grad_dz", "_grad_gamma"):
@@ -439,14 +351,6 @@ def _make_active_op(active: int):
         lambda g, *a: g.new_empty((12, g.shape[-1]), dtype=torch.float32)
     )
 
-    def setup(ctx, inputs, output):
-        ctx.save_for_backward(*inputs[1:14])
-        ctx.active = active
-
-    def backward(ctx, grad_out):
-        return _tri12_grads(ctx, grad_out)
-
-    torch.library.register_autograd(f"jit_thc::{name}", backward, setup_context=setup)
     return getattr(torch.ops.jit_thc, name)
 
 
@@ -550,7 +454,7 @@ torch.library.register_autograd(all_base_b4_12_traceable, _backward_all_base, se
 @torch.library.custom_op("jit_thc::all_base_b4_12_split_traceable", mutates_args=())
 def all_base_b4_12_split_traceable(x0: Tensor, alpha_stack: Tensor) -> list[Tensor]:
     """The L bases R_{alpha_l}(x0) as separate [B,M,C] tensors (one pass over x0)."""
-    return _bases(x0, alpha_stack, stacked=False)
+    _refuse(x0)
 
 
 @_fake(all_base_b4_12_split_traceable)
@@ -573,22 +477,19 @@ def _(x0: Tensor, grad_base: Tensor) -> Tensor:
     return x0.new_empty((grad_base.shape[0], x0.shape[3], K), dtype=torch.float32)
 
 
-def _backward_all_base_split(ctx, *grads):
-    # local_thc_triton_kernels.py:2655-2663
-    if len(grads) == 1 and isinstance(grads[0], (list, tuple)):
-        grads = tuple(grads[0])
-    x0, alpha_stack = ctx.saved_tensors
-    ref = next(g for g in grads if g is not None)
-    grad_base = torch.stack([g.contiguous() if g is not None else torch.zeros_like(ref) for g in grads], dim=0)
-    need = ctx.needs_input_grad
-    grad_x = all_base_b4_12_grad_x_traceable(grad_base, alpha_stack) if need[0] else None
-    grad_alpha = all_base_b4_12_split_grad_alpha_traceable(x0, grad_base).to(alpha_stack.dtype) if need[1] else None
-    return grad_x, grad_alpha
+@torch.library.custom_op("jit_thc::all_base_backward", mutates_args=())
+def all_base_backward(
+    x0: Tensor, grads: list[Tensor], alpha_stack: Tensor, need_x: bool, need_alpha: bool
+) -> tuple[Tensor, Tensor]:
+    """(sum_l R_{alpha_l}^T(grads[l]) as [B,H,H,C], fp32 [L,C,16] of sum_{b,m} x0 grads[l]): both gradients of the
+    bases from the L separate gradients, an empty tensor for one that is not needed."""
+    _refuse(x0)
 
 
-torch.library.register_autograd(
-    all_base_b4_12_split_traceable, _backward_all_base_split, setup_context=_setup_all_base_ctx
-)
+@_fake(all_base_backward)
+def _(x0: Tensor, grads: list[Tensor], alpha_stack: Tensor, need_x: bool, need_alpha: bool):
+    gx = torch.empty_like(x0) if need_x else x0.new_empty((0,))
+    return gx, x0.new_empty((len(grads), x0.shape[3], K) if need_alpha else (0,), dtype=torch.float32)
 
 
 # ---------------------------------------------------------------------------
