@@ -60,6 +60,8 @@ EXPORTS = (
     "lthc_cast_many",
     "lthc_swiglu",
     "lthc_swiglu_bwd",
+    "lthc_linear_weight_grad_workspace_bytes",
+    "lthc_linear_weight_grad",
     "lthc_gate_add_norm_modulate_fwd",
     "lthc_gate_add_norm_modulate_bwd_workspace_bytes",
     "lthc_gate_add_norm_modulate_bwd",
@@ -133,6 +135,7 @@ def load() -> ctypes.CDLL:
         "lthc_cast_many": [vp, vp, i64, vp, ci, vp],
         "lthc_swiglu": [vp, ci, vp, i64, i64, vp],
         "lthc_swiglu_bwd": [vp, vp, ci, vp, i64, i64, vp],
+        "lthc_linear_weight_grad": [vp, vp, ci, vp, vp, i64, i64, i64, vp, sz, vp],
         "lthc_gate_add_norm_modulate_bwd": [
             vp, vp, vp, vp, vp, ci, vp, ci, vp, i64, vp, vp, vp, vp, vp, vp, ci, i64, i64, i64, ctypes.c_float, vp, sz,
             vp,
@@ -182,7 +185,7 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name + "_workspace_bytes")
         fn.argtypes = [i64, i64, i64, i64]
         fn.restype = sz
-    for name in ("lthc_gate_add_norm_modulate_bwd", "lthc_gate_residual_bwd"):
+    for name in ("lthc_gate_add_norm_modulate_bwd", "lthc_gate_residual_bwd", "lthc_linear_weight_grad"):
         fn = getattr(lib, name + "_workspace_bytes")
         fn.argtypes = [i64, i64, i64]
         fn.restype = sz

@@ -13,3 +13,5 @@
 #include "attention.inc"
 // The attention's backward.
 #include "attention_backward.inc"
+// Weight and bias gradients of the linear layers over many rows.
+#include "linear_weight_grad.inc"

@@ -893,6 +893,25 @@ std::tuple<Tensor, Tensor> gate_residual_backward_cuda(const Tensor& grad_, cons
   return {ggate, gm};
 }
 
+// (gW [N, K], gb [N] or an empty tensor) of a linear layer for the output gradient [..., N] and the input [..., K].
+std::tuple<Tensor, Tensor> linear_weight_grad_cuda(const Tensor& grad_, const Tensor& x_, bool need_bias) {
+  on_gpu(grad_, x_);
+  TORCH_CHECK_VALUE(grad_.dim() >= 1 && grad_.dim() == x_.dim() && grad_.sizes().slice(0, grad_.dim() - 1) ==
+                                                                      x_.sizes().slice(0, x_.dim() - 1),
+                    "grad [..., N] and x [..., K] expected, got ", shape(grad_), " and ", shape(x_));
+  TORCH_CHECK_VALUE(grad_.scalar_type() == x_.scalar_type(), "grad and x must have one dtype, got ", grad_.scalar_type(),
+                    ", ", x_.scalar_type());
+  const Tensor grad = prep16(grad_), x = prep16(x_);
+  const int64_t n = grad.size(-1), k = x.size(-1), m = n ? grad.numel() / n : 0;
+  Tensor gw = at::empty({n, k}, grad.options()), gb = at::empty({need_bias ? n : 0}, grad.options());
+  const Tensor ws = workspace(lthc_linear_weight_grad_workspace_bytes(m, n, k), grad);
+  const Launch l(grad);
+  check(lthc_linear_weight_grad(data(grad), data(x), code(grad), data(gw), need_bias ? data(gb) : nullptr, m, n, k, data(ws),
+                                ws.numel(), l.stream),
+        "lthc_linear_weight_grad");
+  return {gw, gb};
+}
+
 std::tuple<Tensor, Tensor, Tensor> block_tail_cuda(const Tensor& z_, const Tensor& a_, const Tensor& gate,
                                                    const Tensor& m_, const Tensor& gamma, const Tensor& weight,
                                                    const Tensor& shift, const Tensor& scale, double eps) {
@@ -980,6 +999,8 @@ LTHC_OP(op_ganm_backward, "gate_add_norm_modulate_backward",
                                                                    const Tensor&, const Tensor&, double))
 LTHC_OP(op_gres, "gate_residual", Tensor(const Tensor&, const Tensor&, const Tensor&))
 LTHC_OP(op_gres_backward, "gate_residual_backward", std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&))
+
+LTHC_OP(op_linear_weight_grad, "linear_weight_grad", std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, bool))
 
 using BelowAutograd = at::AutoDispatchBelowADInplaceOrView;
 
@@ -1447,6 +1468,36 @@ struct GresFn : torch::autograd::Function<GresFn> {
   }
 };
 
+// A linear layer whose weight and bias gradients come from one pass over the rows (linear_weight_grad).  The forward
+// and the input's gradient are torch's own products.  Where a graph of the backward is built, or the kernel does not
+// take the shapes, the weight's gradient is the product torch's linear has.
+struct LinearFn : torch::autograd::Function<LinearFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const std::optional<Tensor>& bias) {
+    BelowAutograd below;
+    ctx->save_for_backward({x, weight});
+    ctx->saved_data["bias"] = bias.has_value() && bias->defined();
+    return at::linear(x, weight, bias);
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &weight = saved[1], &g = grads[0];
+    const bool need_w = ctx->needs_input_grad(1);
+    const bool need_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2);
+    Tensor gx, gw, gb;
+    if (ctx->needs_input_grad(0)) gx = at::matmul(g, weight);
+    if (need_w && !at::GradMode::is_enabled() && x.numel() > 0 && x.size(-1) % 8 == 0 && g.size(-1) % 8 == 0) {
+      BelowAutograd below;
+      std::tie(gw, gb) = op_linear_weight_grad().call(g, x, need_b);
+      if (!need_b) gb = Tensor();
+    } else if (need_w || need_b) {
+      const Tensor g2 = g.reshape({-1, g.size(-1)});
+      if (need_w) gw = g2.t().matmul(x.reshape({-1, x.size(-1)}));
+      if (need_b) gb = g2.sum(0);
+    }
+    return {gx, gw, gb};
+  }
+};
+
 // ---- AutogradCUDA kernels: record a node, or go straight below autograd
 Tensor read_autograd(const Tensor& x, const Tensor& w) {
   if (recording(x, w)) return ReadFn::apply(x, w);
@@ -1567,6 +1618,10 @@ std::tuple<Tensor, Tensor> read_with_residual(const Tensor& x, const Tensor& wei
   return pair(OpenFn::apply(x, weight));
 }
 
+Tensor linear(const Tensor& x, const Tensor& weight, const std::optional<Tensor>& bias) {
+  return LinearFn::apply(x, weight, bias);
+}
+
 std::vector<Tensor> lazy_workspace_step(const Tensor& z, const Tensor& dz, const Tensor& gamma, bool split) {
   return StepFn::apply(z, dz, gamma, split);
 }
@@ -1575,6 +1630,7 @@ std::vector<Tensor> lazy_workspace_step(const Tensor& z, const Tensor& dz, const
 
 TORCH_LIBRARY_FRAGMENT(jit_thc, m) {
   m.def("read_with_residual(Tensor x, Tensor weight) -> (Tensor, Tensor)", read_with_residual);
+  m.def("linear(Tensor x, Tensor weight, Tensor? bias) -> Tensor", linear);
   m.def("lazy_workspace_step(Tensor z, Tensor dz, Tensor gamma, bool split) -> Tensor[]", lazy_workspace_step);
 }
 
@@ -1624,6 +1680,7 @@ TORCH_LIBRARY_IMPL(jit_thc, CUDA, m) {
   m.impl("gate_add_norm_modulate_backward", gate_add_norm_modulate_backward_cuda);
   m.impl("gate_residual", gate_residual_cuda);
   m.impl("gate_residual_backward", gate_residual_backward_cuda);
+  m.impl("linear_weight_grad", linear_weight_grad_cuda);
   m.impl("block_tail", block_tail_cuda);
 }
 

@@ -40,13 +40,21 @@ def modulate(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor) -> torch
 class CastLinear(nn.Linear):
     """nn.Linear that, while the model's forward has converted every weight in one batched launch
     (``BatchedWeightCast._converted_weights``), multiplies by that (weight, bias) pair: the values
-    autocast's own per-layer conversion would give.  Parameters and state-dict names are nn.Linear's."""
+    autocast's own per-layer conversion would give.  In a 16-bit training forward over many rows its weight and bias
+    gradients come from one HIP pass (``ops_branch.linear``).  Parameters and state-dict names are nn.Linear's."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         cast = self.__dict__.get("_cast")
         if cast is not None:
             return F.linear(x, cast[0], cast[1])
-        return super().forward(x)
+        y = ops_branch.linear(x, self.weight, self.bias)
+        return y if y is not None else super().forward(x)
+
+
+def _linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """F.linear, its weight and bias gradients from one HIP pass where ops_branch.linear applies."""
+    y = ops_branch.linear(x, weight, bias)
+    return y if y is not None else F.linear(x, weight, bias)
 
 
 class RMSNorm(nn.Module):
@@ -167,8 +175,8 @@ class BottleneckPatchEmbedNHWC(nn.Module):
         patches = _patch_rows(x, self.patch_size[0], self.grid_size)
         cast = self.__dict__.get("_cast")
         w1, w2, b2 = cast if cast is not None else (self.proj1.weight, self.proj2.weight, self.proj2.bias)
-        h = F.linear(patches, w1.view(self.proj1.out_channels, -1))
-        return F.linear(h, w2.view(self.proj2.out_channels, -1), b2)
+        h = _linear(patches, w1.view(self.proj1.out_channels, -1))
+        return _linear(h, w2.view(self.proj2.out_channels, -1), b2)
 
     def cast_targets(self) -> list[torch.Tensor] | None:
         """The tensors forward() takes, in order, from a batched conversion set as ``_cast`` (None: no such form)."""
@@ -201,7 +209,7 @@ class DirectPatchEmbedNHWC(nn.Module):
         patches = _patch_rows(x, self.patch_size[0], self.grid_size)
         cast = self.__dict__.get("_cast")
         w, bias = cast if cast is not None else (self.proj.weight, self.proj.bias)
-        return F.linear(patches, w.view(self.proj.out_channels, -1), bias)
+        return _linear(patches, w.view(self.proj.out_channels, -1), bias)
 
     def cast_targets(self) -> list[torch.Tensor] | None:
         """The tensors forward() takes, in order, from a batched conversion set as ``_cast`` (None: no such form)."""

@@ -361,6 +361,17 @@ int lthc_qk_norm_rope_attention_bwd(const void* qkv, const void* grad, int x_dty
                                     size_t workspace_bytes, void* stream);
 
 /*
+ * WEIGHT AND BIAS GRADIENT OF A LINEAR LAYER (no reference op: autograd of the
+ * model's nn.Linear layers).  For g [M, N] and x [M, K] (x_dtype, bf16 or
+ * fp16): gw[n,k] = sum_m g[m,n] x[m,k] and gb[n] = sum_m g[m,n] (gb may be
+ * NULL), fp32 sums in a fixed order rounded once to x_dtype.  N and K
+ * multiples of 8; every pointer 16-byte aligned.
+ */
+size_t lthc_linear_weight_grad_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int lthc_linear_weight_grad(const void* g, const void* x, int x_dtype, void* gw, void* gb, int64_t M, int64_t N,
+                            int64_t K, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * DECODER HEAD (no reference op: FinalLayerSharedAdaLN.forward and
  * unpatchify, local_thc.py:865-873 and :972-980, are eager torch).  For the
  * materialised x [B, h*w, C] (x_dtype bf16 or fp16):

@@ -7,6 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from flowmatching_lthc_amd import model as M
 from flowmatching_lthc_amd import ops
 from flowmatching_lthc_amd import ops_branch as OB
 
@@ -64,7 +65,8 @@ def test_attention_backward(N, H, dtype, tdt, wdt):
     assert e.shape == (0, N, 3, H, 64) and dw.abs().max().item() == 0.0
 
 
-UNIT = {torch.float32: 2.0**-24, torch.bfloat16: 2.0**-9, torch.float16: 2.0**-12}
+# RMS-size of one rounding of a result, relative to it: half the unit roundoff
+UNIT = {torch.float32: 2.0**-25, torch.bfloat16: 2.0**-9, torch.float16: 2.0**-12}
 
 
 def check_grads(names, ours, eager, exact, dtype):
@@ -179,3 +181,66 @@ def test_qk_norm_rope_backward(B, N, H, dtype, tdt, wdt):
     eager = grads_of(lambda *t: OB.qk_norm_rope_eager(*t, cos, sin, 1e-6), tensors, (gq, gk))
     check_grads(("qkv", "q weight", "k weight"), ours, eager, grads_of(exact, tensors, (gq, gk), torch.float64), dtype)
     assert ours[0][:, :, 2].abs().max().item() == 0.0
+
+
+# ends of the 256 x 128 tile and of the 32-row stage, one stage, an odd number of stages, parts that end inside a stage,
+# fewer tiles and more tiles than blocks fit at once
+@pytest.mark.parametrize("rows,N,K", [(1, 8, 8), (33, 264, 136), (96, 256, 128), (1000, 48, 768), (4097, 520, 392), (600, 4096, 2048)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_linear_weight_grad(rows, N, K, dtype):
+    print(f"case linear weight grad rows={rows} N={N} K={K} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(rows + N)
+    g, x = torch.randn((rows, N), generator=gen).to(DEV, dtype), torch.randn((rows, K), generator=gen).to(DEV, dtype)
+    gw, gb = OB.linear_weight_grad(g, x, True)
+    for got, ref, name in ((gw, g.double().t() @ x.double(), "weight"), (gb, g.double().sum(0), "bias")):
+        # one rounding of an fp32 sum, u = 2^-8 (bf16: 8 significant bits) or 2^-11 (fp16: 11):
+        # |d| <= u |ref| + 2^-20 sum |terms| (fp32 sums of up to `rows` terms in any order)
+        u = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+        terms = g.double().abs().t() @ x.double().abs() if name == "weight" else g.double().abs().sum(0)
+        tiny = 2.0**-25 if dtype == torch.float16 else 0.0  # half of fp16's smallest step
+        assert ((got.double() - ref).abs() <= u * ref.abs() * (1 + 2.0**-10) + 2.0**-20 * terms + tiny).all(), name
+    none = OB.linear_weight_grad(g, x, False)
+    assert torch.equal(none[0], gw) and none[1].numel() == 0
+
+
+def test_linear_layer_routes():
+    """The layer's training route against torch's linear: values, gradients under autocast and in 16 bits, without a
+    bias, a frozen weight, a graph of the backward, a batch of gradients; and the calls that stay torch's own."""
+    print("case linear layer routes", flush=True)
+    lin, ref = M.CastLinear(64, 136).to(DEV), torch.nn.Linear(64, 136).to(DEV)
+    ref.load_state_dict(lin.state_dict())
+    x = torch.randn((4, 200, 64), generator=torch.Generator().manual_seed(0)).to(DEV)
+    g = torch.randn((4, 200, 136), generator=torch.Generator().manual_seed(1)).to(DEV)
+
+    def grads(layer, x, g, amp):
+        xl = x.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=amp):
+            y = layer(xl)
+        return [y, *torch.autograd.grad(y, [xl, *[p for p in layer.parameters() if p.requires_grad]], g.to(y.dtype))]
+
+    def same(a, b):
+        for p, q in zip(a, b, strict=True):
+            assert p.dtype == q.dtype and p.shape == q.shape and rel(p, q) <= 4e-3
+
+    assert OB.linear(x.bfloat16(), lin.weight.bfloat16(), None) is not None
+    same(grads(lin, x, g, True), grads(ref, x, g, True))  # fp32 weights under autocast
+    same(grads(lin.bfloat16(), x.bfloat16(), g, False), grads(ref.bfloat16(), x.bfloat16(), g, False))
+    xl = x.bfloat16().requires_grad_()
+    y = lin(xl)
+    (a,) = torch.autograd.grad(y, lin.weight, torch.stack((g, 2 * g)).bfloat16(), is_grads_batched=True, retain_graph=True)
+    assert rel(a[1], 2 * a[0]) <= 4e-3
+    second = []
+    for layer in (lin, ref):  # a graph of the backward
+        y = layer(xl)
+        (gw,) = torch.autograd.grad(y, layer.weight, g.bfloat16(), create_graph=True)
+        second.append(torch.autograd.grad(gw.float().square().sum(), xl)[0])
+    assert rel(*second) <= 1e-2
+    lin.weight.requires_grad_(False)
+    assert OB.linear(xl, lin.weight, lin.bias) is None and lin(xl).requires_grad
+    lin.weight.requires_grad_(True)
+    w = lin.weight.detach()
+    assert OB.linear(xl[:1, :100], lin.weight, None) is None and OB.linear(x, lin.weight, None) is None
+    out = torch.func.grad(lambda t: torch.nn.functional.linear(t, w).float().sum())(x.bfloat16())
+    assert rel(torch.func.grad(lambda t: lin(t).float().sum())(x.bfloat16()), out) <= 1e-6
+    with torch.no_grad():
+        assert OB.linear(xl, lin.weight, None) is None
