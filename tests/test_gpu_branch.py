@@ -245,6 +245,29 @@ def test_qk_norm_rope_attention_matches_exact(dtype, N, H):
     assert (eager.double().cpu() - ref).abs().max().item() <= max(2 * e_sdpa, u * vmax)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N", [64, 128, 192, 256])
+def test_qk_norm_rope_attention_table_and_weight_formats(dtype, N):
+    """Every instance of the kernel (token blocks x table format), with weights in either format: the tables and weights
+    that 16 bits hold give the same output bit for bit when they come in fp32, and each element is within one rounding
+    of the probabilities and one of the output of softmax attention in float64 (the bound of the test above)."""
+    print(f"case formats dtype={dtype} N={N}", flush=True)
+    gen = torch.Generator().manual_seed(N)
+    qkv = (torch.randn((3, N, 3, 3, 64), generator=gen) * 2.0).to(DEV, dtype)
+    qw, kw = ((torch.randn(64, generator=gen) * 0.2 + 1).to(DEV, dtype) for _ in range(2))
+    cos, sin = (t.to(dtype) for t in random_rope_tables(N, gen))
+    o = OB.qk_norm_rope_attention(qkv, qw, kw, cos, sin, 1e-6)
+    for w in ((qw, kw), (qw.float(), kw.float())):
+        for tab in ((cos, sin), (cos.float(), sin.float())):
+            assert torch.equal(OB.qk_norm_rope_attention(qkv, *w, *tab, 1e-6), o)
+    q, k = OB.qk_norm_rope(qkv, qw, kw, cos, sin, 1e-6)
+    v = qkv[:, :, 2]
+    ref = attention_exact(q, k, v)
+    u = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    bad = ((o.double().cpu() - ref).abs() > u * (v.double().abs().max().item() + ref.abs())).sum().item()
+    assert bad == 0, f"{bad} elements beyond one rounding"
+
+
 def test_qk_norm_rope_attention_gradients_and_errors():
     """The backward (recomputed through the eager q/k norm + RoPE sequence, the attention itself in fp32 products)
     matches autograd of the eager sequence to 1e-2 of each gradient's scale; unsupported shapes and dtypes raise
