@@ -1091,13 +1091,15 @@ struct WriteAddFn : torch::autograd::Function<WriteAddFn> {
 };
 
 // (x, Z0 = R(x)) as one node, x returned as a view of itself: its gradient and Z0's arrive together, and
-// dX = g_x + R^T gZ0 is one pass.
+// dX = g_x + R^T gZ0 is one pass.  The alias is made outside the guard: autograd then knows it as a view that shares
+// the saved x's version counter, and refuses an in-place change of it.
 struct OpenFn : torch::autograd::Function<OpenFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight) {
+    const Tensor alias = x.view_as(x);
     BelowAutograd below;
     ctx->save_for_backward({x, weight});
     ctx->set_materialize_grads(false);  // an unused output's gradient stays undefined
-    return {x.view_as(x), op_read().call(x, weight)};
+    return {alias, op_read().call(x, weight)};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     BackwardScope scope;
@@ -1200,13 +1202,15 @@ struct RecurFn : torch::autograd::Function<RecurFn> {
 // split Z_{l+1}'s two, arrive together and one recurrence-backward launch sums them.
 struct StepFn : torch::autograd::Function<StepFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& z, const Tensor& dz, const Tensor& gamma, bool split) {
-    BelowAutograd below;
     ctx->save_for_backward({dz, gamma});
     ctx->saved_data["z"] = static_cast<int64_t>(z.scalar_type());
     ctx->saved_data["split"] = split;
     ctx->set_materialize_grads(false);  // an unused Z_{l+1} (the last step's) skips the recurrence backward
-    const Tensor zn = op_recur().call(z, dz, gamma);
-    if (split) return {zn, zn.view_as(zn), dz.view_as(dz)};
+    const Tensor zn = [&] {
+      BelowAutograd below;
+      return op_recur().call(z, dz, gamma);
+    }();
+    if (split) return {zn, zn.view_as(zn), dz.view_as(dz)};  // views for autograd, as OpenFn's
     return {zn, dz.view_as(dz)};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
