@@ -1,5 +1,5 @@
 // The jit_thc operators on GPU tensors: argument checks, output allocation and the launch through include/lthc.h for
-// the CUDA dispatch key, and the autograd formulas for AutogradCUDA.  The schemas and the fake (meta) kernels are
+// the CUDA dispatch key, and the autograd formulas of every device.  The schemas and the fake (meta) kernels are
 // registered from Python (ops.py, ops_branch.py, ops_triangular.py), which also refuse tensors of other devices; the
 // reference's formulas each node follows are cited there.
 //
@@ -1502,7 +1502,7 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
   }
 };
 
-// ---- AutogradCUDA kernels: record a node, or go straight below autograd
+// ---- autograd kernels: record a node, or go straight below autograd
 Tensor read_autograd(const Tensor& x, const Tensor& w) {
   if (recording(x, w)) return ReadFn::apply(x, w);
   BelowAutograd below;
@@ -1688,7 +1688,9 @@ TORCH_LIBRARY_IMPL(jit_thc, CUDA, m) {
   m.impl("block_tail", block_tail_cuda);
 }
 
-TORCH_LIBRARY_IMPL(jit_thc, AutogradCUDA, m) {
+// The nodes hold no device code: meta tensors, fake ones of any device and CPU tensors (whose kernels refuse them, or are
+// registered by a program) get the same formulas.
+static void autograd_kernels(torch::Library& m) {
   m.impl("local_write_traceable", read_autograd);
   m.impl("local_read_traceable", write_autograd);
   m.impl("local_read_add_traceable", write_add_autograd);
@@ -1707,3 +1709,7 @@ TORCH_LIBRARY_IMPL(jit_thc, AutogradCUDA, m) {
   m.impl("gate_add_norm_modulate", ganm_autograd);
   m.impl("gate_residual", gres_autograd);
 }
+
+TORCH_LIBRARY_IMPL(jit_thc, AutogradCUDA, m) { autograd_kernels(m); }
+TORCH_LIBRARY_IMPL(jit_thc, AutogradMeta, m) { autograd_kernels(m); }
+TORCH_LIBRARY_IMPL(jit_thc, AutogradCPU, m) { autograd_kernels(m); }

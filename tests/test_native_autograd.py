@@ -9,6 +9,8 @@ import pytest
 import torch
 
 from flowmatching_lthc_amd import ops
+from flowmatching_lthc_amd import ops_branch as OB
+from flowmatching_lthc_amd import ops_triangular as OT
 
 
 def cells(x):
@@ -114,3 +116,52 @@ def test_interface_nodes_give_the_gradients_of_the_plain_sequence():
     )
     for a, b in zip(got, want):
         torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
+# ---------------------------------------------------------------------------
+# devices
+# ---------------------------------------------------------------------------
+def meta(*shape, dtype=torch.float32):
+    return torch.empty(shape, device="meta", dtype=dtype, requires_grad=True)
+
+
+def meta_cases():
+    x, w, z, dz, row, rows = meta(2, 8, 8, 8), meta(8, 16), meta(2, 4, 8), meta(2, 4, 8), meta(8), meta(2, 8)
+    qkv, tables = meta(2, 64, 3, 2, 64, dtype=torch.bfloat16), meta(64, 64)
+    norm, stack = meta(64), meta(3, 8, 16)
+    twelve = [meta(2, 4, 8) for _ in range(12)], [meta(8, 16) for _ in range(12)]
+    qk = (qkv, norm, norm, tables.detach(), tables.detach(), 1e-6)
+    return {
+        "read": (ops.local_write_traceable, (x, w)),
+        "write": (ops.local_read_traceable, (z, w)),
+        "write_add": (ops.local_read_add_traceable, (z, w, x)),
+        "read_with_residual": (ops.read_with_residual, (x, w)),
+        "step": (ops.lazy_workspace_step, (z, dz, row, True)),
+        "update": (ops.lazy_workspace_update, (z, dz, row)),
+        "final_list": (lambda x, d, b: ops.final_accumulate_list(x, [d], [b]), (x, dz, w)),
+        "final_12": (lambda x, *rest: ops.final_accumulate_b4_12_traceable(x, *rest), (x, *twelve[0], *twelve[1])),
+        "gamma_rounded": (lambda a, b: ops.lazy_gamma_rounded(a, [b], torch.bfloat16), (w, meta(8, 16))),
+        "bases": (OT.all_base_b4_12_split_traceable, (x, stack)),
+        "tri_list": (lambda z, d, g: OT.triangular_accumulate_list(z, [d], g), (z, dz, meta(1, 8))),
+        "tri_12": (OT.triangular_accumulate_b4_12_ptr_traceable, (z, *twelve[0], meta(12, 8))),
+        "tri_active": (OT.triangular_accumulate_b4_12_ptr_active_traceable_ops[4], (z, *twelve[0], meta(12, 8))),
+        "norm_modulate": (ops.norm_modulate, (z, row, rows, rows, 1e-6)),
+        "qk_norm_rope": (OB.qk_norm_rope, qk),
+        "attention": (OB.qk_norm_rope_attention, qk),
+        "swiglu": (OB.swiglu, (meta(2, 16),)),
+        "gate_add_norm_modulate": (OB.gate_add_norm_modulate, (z, dz, rows, row, rows, rows, 1e-6)),
+        "gate_residual": (OB.gate_residual, (z, rows, dz)),
+    }
+
+
+@pytest.mark.parametrize("name", meta_cases())
+def test_gradients_of_meta_tensors(name):
+    """Shapes can be propagated through forward and backward without a device, as through torch's own operators."""
+    f, args = meta_cases()[name]
+    outs = f(*args)
+    outs = [outs] if isinstance(outs, torch.Tensor) else list(outs)
+    leaves = list({id(a): a for a in args if isinstance(a, torch.Tensor) and a.requires_grad}.values())
+    grads = torch.autograd.grad(outs, leaves, [torch.empty_like(o) for o in outs], allow_unused=True)
+    assert any(g is not None for g in grads)
+    for g, a in zip(grads, leaves):
+        assert g is None or (g.shape, g.dtype, g.device) == (a.shape, a.dtype, a.device)
