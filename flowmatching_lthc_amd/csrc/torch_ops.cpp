@@ -1460,10 +1460,10 @@ struct GresFn : torch::autograd::Function<GresFn> {
     Tensor ggate, gm;
     const bool need_gate = ctx->needs_input_grad(1), need_m = ctx->needs_input_grad(2);
     if (need_gate || need_m) {
-      if (m.sym_size(2) <= kNormMaxChannels) {
-        DetachedScope scope;
+      if (!at::GradMode::is_enabled() && m.sym_size(2) <= kNormMaxChannels) {
+        BelowAutograd below;
         std::tie(ggate, gm) = op_gres_backward().call(grad, gate, m);
-      } else {  // wider than the kernel's rows
+      } else {  // a graph of the backward is built, or wider than the kernel's rows
         if (need_gate) ggate = as_dtype(at::sum(as_dtype(grad * m, at::kFloat), 1), gate.scalar_type());
         if (need_m) gm = grad * gate.unsqueeze(1);
       }

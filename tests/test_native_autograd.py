@@ -43,6 +43,8 @@ KERNELS = {
     "lazy_workspace_update": lambda z, dz, gamma: z + gamma * dz,
     "lazy_workspace_update_backward": recur_backward,
     "lazy_workspace_update_backward_sum": lambda g, b, dz, gamma, add=None: (g + b, *recur_backward(g + b, dz, gamma, add)),
+    "gate_residual": OB.gate_residual_eager,
+    "gate_residual_backward": lambda g, gate, m: ((g * m).sum(1), g * gate.unsqueeze(1)),
 }
 
 
@@ -116,6 +118,21 @@ def test_interface_nodes_give_the_gradients_of_the_plain_sequence():
     )
     for a, b in zip(got, want):
         torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
+# ---------------------------------------------------------------------------
+# graphs of the backward
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("C", [8, 2056])  # within the backward kernel's widths, and beyond
+def test_second_derivative_of_gate_residual(C):
+    """create_graph: the gradients of the gate and m are products of both, as in the plain sequence."""
+    leaves = [leaf((2, 4, C), 0), leaf((2, C), 1), leaf((2, 4, C), 2)]
+    results = []
+    for f in (OB.gate_residual, OB.gate_residual_eager):
+        first = torch.autograd.grad(f(*leaves).pow(2).sum(), leaves, create_graph=True)
+        results.append([*first, *torch.autograd.grad(sum(g.square().sum() for g in first), leaves)])
+    for a, b in zip(*results):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-4)
 
 
 # ---------------------------------------------------------------------------
