@@ -958,6 +958,8 @@ LTHC_OP(op_final_12, "final_accumulate_b4_12_traceable", Tensor(const Tensor&, L
 LTHC_OP(op_final_backward, "final_accumulate_backward", std::tuple<Tensor, Tensor>(const Tensor&, TensorList, TensorList))
 LTHC_OP(op_list_grad_dz, "final_accumulate_list_grad_dz", std::vector<Tensor>(const Tensor&, TensorList))
 LTHC_OP(op_list_grad_beta, "final_accumulate_list_grad_beta", Tensor(const Tensor&, TensorList))
+LTHC_OP(op_12_grad_dz, "final_accumulate_b4_12_grad_dz_ptr", Tensor(const Tensor&, LTHC_TYPES12))
+LTHC_OP(op_12_grad_beta, "final_accumulate_b4_12_grad_beta_ptr", Tensor(const Tensor&, LTHC_TYPES12))
 LTHC_OP(op_recur, "lazy_workspace_update", Tensor(const Tensor&, const Tensor&, const Tensor&))
 LTHC_OP(op_recur_backward, "lazy_workspace_update_backward",
         std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&, const std::optional<Tensor>&))
@@ -970,6 +972,8 @@ LTHC_OP(op_gamma_rounded_backward, "lazy_gamma_rounded_backward",
 LTHC_OP(op_all_base_split, "all_base_b4_12_split_traceable", std::vector<Tensor>(const Tensor&, const Tensor&))
 LTHC_OP(op_all_base_backward, "all_base_backward",
         std::tuple<Tensor, Tensor>(const Tensor&, TensorList, const Tensor&, bool, bool))
+LTHC_OP(op_all_base_grad_x, "all_base_b4_12_grad_x", Tensor(const Tensor&, const Tensor&))
+LTHC_OP(op_all_base_grad_alpha, "all_base_b4_12_split_grad_alpha", Tensor(const Tensor&, const Tensor&))
 LTHC_OP(op_tri_list, "triangular_accumulate_list", Tensor(const Tensor&, TensorList, const Tensor&))
 LTHC_OP(op_ws_backward, "ws_accumulate_backward",
         std::tuple<std::vector<Tensor>, Tensor>(const Tensor&, TensorList, const Tensor&, c10::SymInt, bool))
@@ -1037,6 +1041,19 @@ bool any_needed(AutogradContext* ctx, size_t from, size_t count) {
   for (size_t i = 0; i < count; ++i)
     if (ctx->needs_input_grad(from + i)) return true;
   return false;
+}
+
+// Whether a gradient holds a batch of them (is_grads_batched, vmap).  Torch then runs an op once per sample by itself,
+// except for ops over tensor lists, which those nodes replace by ops over plain tensors.
+bool batched(TensorList ts) {
+  const c10::DispatchKeySet keys({c10::DispatchKey::Batched, c10::DispatchKey::FuncTorchBatched});
+  for (const Tensor& t : ts)
+    if (t.key_set().has_any(keys)) return true;
+  return false;
+}
+
+Tensor call_12(const c10::TypedOperatorHandle<Tensor(const Tensor&, LTHC_TYPES12)>& op, const Tensor& t, TensorList l) {
+  return op.call(t, l[0], l[1], l[2], l[3], l[4], l[5], l[6], l[7], l[8], l[9], l[10], l[11]);
 }
 
 struct ReadFn : torch::autograd::Function<ReadFn> {
@@ -1122,7 +1139,13 @@ variable_list final_grads(AutogradContext* ctx, const Tensor& grad, TensorList d
   variable_list out(1 + 2 * L);
   out[0] = grad_out;
   Tensor gb;
-  if (want_dz && want_beta) {
+  if (L == 12 && batched(grad_out)) {
+    if (want_dz) {
+      const auto parts = call_12(op_12_grad_dz(), grad_out, betas).unbind(0);
+      for (size_t i = 0; i < L; ++i) out[1 + i] = parts[i];
+    }
+    if (want_beta) gb = call_12(op_12_grad_beta(), grad_out, dzs);
+  } else if (want_dz && want_beta) {
     Tensor gdz;
     std::tie(gdz, gb) = op_final_backward().call(grad_out, dzs, betas);
     const auto parts = gdz.unbind(0);
@@ -1272,7 +1295,14 @@ struct AllBaseSplitFn : torch::autograd::Function<AllBaseSplitFn> {
     const auto saved = ctx->get_saved_variables();
     const Tensor &x0 = saved[0], &alpha_stack = saved[1];
     const bool need_x = ctx->needs_input_grad(0), need_a = ctx->needs_input_grad(1);
-    auto [gx, ga] = op_all_base_backward().call(x0, grads, alpha_stack, need_x, need_a);
+    Tensor gx, ga;
+    if (batched(grads)) {
+      const Tensor base = at::stack(grads);
+      if (need_x) gx = op_all_base_grad_x().call(base, alpha_stack);
+      if (need_a) ga = op_all_base_grad_alpha().call(x0, base);
+    } else {
+      std::tie(gx, ga) = op_all_base_backward().call(x0, grads, alpha_stack, need_x, need_a);
+    }
     return {need_x ? gx : Tensor(), need_a ? as_dtype(ga, alpha_stack.scalar_type()) : Tensor()};
   }
 };

@@ -26,8 +26,8 @@ activation dtype), registered as a ``jit_thc`` custom op:
 
 Every op but block_tail (inference only) has a backward kernel of its own,
 ``jit_thc::<op>_backward``, one HIP pass that recomputes what it needs from the
-op's inputs and gives the gradients of the eager sequence.  Batched gradients
-(vmap) differentiate the eager sequence itself.
+op's inputs and gives the gradients of the eager sequence.  For batched
+gradients (is_grads_batched, vmap) torch runs that pass once per sample.
 """
 
 from __future__ import annotations
@@ -43,7 +43,7 @@ QK_HEAD_DIM = 64
 
 
 # ---------------------------------------------------------------------------
-# eager restatements (the tests' reference; batched gradients differentiate them)
+# eager restatements: what each kernel's values and gradients are compared with
 # ---------------------------------------------------------------------------
 def _rms_norm_eager(x: Tensor, weight: Tensor, eps: float) -> Tensor:
     xf = x.float()

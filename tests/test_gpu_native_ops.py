@@ -103,6 +103,41 @@ def test_graph_of_the_backward_through_the_read():
     assert (second[0] - second[1]).abs().max() <= 1e-5 * second[1].abs().max()
 
 
+def batched_cases():
+    z, a, m, w = randn((2, 9, 24), 0), randn((2, 9, 24), 1), randn((2, 9, 24), 2), randn((24,), 3)
+    gate, shift, scale = (randn((2, 24), 4 + i) for i in range(3))
+    qkv, n0, n1, table = randn((2, 6, 3, 2, 64), 7), randn((64,), 8), randn((64,), 9), randn((6, 64), 10)
+    x0, alpha, betas, dzs = inputs(12)
+    return {
+        "norm_modulate": (lambda *t: ops.norm_modulate(*t, 1e-6)[0], (z, w, shift, scale)),
+        "gate_add_norm_modulate": (lambda *t: OB.gate_add_norm_modulate(*t, 1e-6), (z, a, gate, w, shift, scale)),
+        "gate_residual": (OB.gate_residual, (a, gate, m)),
+        "swiglu": (OB.swiglu, (randn((5, 48), 11),)),
+        "qk_norm_rope": (lambda *t: OB.qk_norm_rope(*t, table, table, 1e-6), (qkv, n0, n1)),
+        "bases": (OT.all_base_b4_12_split_traceable, (x0, torch.stack(betas[:3]))),
+        "materialise dz": (lambda *d: ops.final_accumulate_b4_12_traceable(x0, *d, *betas), tuple(dzs)),
+        "materialise beta": (lambda *b: ops.final_accumulate_b4_12_traceable(x0, *dzs, *b), tuple(betas)),
+        "read": (ops.read_with_residual, (x0, alpha)),
+        "step": (lambda *t: ops.lazy_workspace_step(*t, True), (dzs[0], dzs[1], randn((20,), 12))),
+    }
+
+
+@pytest.mark.parametrize("name", ["norm_modulate", "gate_add_norm_modulate", "gate_residual", "swiglu", "qk_norm_rope",
+                                  "bases", "materialise dz", "materialise beta", "read", "step"])  # fmt: skip
+def test_batched_gradients(name):
+    """is_grads_batched gives each sample's own gradients, bit for bit (the same kernels, once per sample)."""
+    print(f"case native ops: batched gradients of {name}", flush=True)
+    f, tensors = batched_cases()[name]
+    ls = [t.detach().requires_grad_() for t in tensors]
+    outs = f(*ls)
+    outs = [outs] if isinstance(outs, torch.Tensor) else list(outs)
+    grads = [randn((3, *o.shape), 20 + i) for i, o in enumerate(outs)]
+    got = torch.autograd.grad(outs, ls, grads, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for a, b in zip(got, torch.autograd.grad(outs, ls, [g[i] for g in grads], retain_graph=True)):
+            assert torch.equal(a[i], b)
+
+
 def test_refusals():
     print("case native ops: refusals", flush=True)
     x, w = randn((1, 8, 8, 8), 0), randn((8, 16), 1)

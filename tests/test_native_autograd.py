@@ -31,6 +31,16 @@ def write(z, w):
     return x.permute(0, 1, 3, 2, 4, 5).reshape(B, 4 * G, 4 * G, C)
 
 
+def weight_grad(high, low):
+    return (cells(high) * low[:, :, None]).sum((0, 1)).t().contiguous()
+
+
+def all_base_backward(x, grads, alphas, need_x, need_alpha):
+    empty = x.new_empty(0)
+    gx = sum(map(write, grads, alphas)) if need_x else empty
+    return gx, torch.stack([weight_grad(x, g) for g in grads]) if need_alpha else empty
+
+
 def recur_backward(g, dz, gamma, add=None):
     return gamma * g + (0 if add is None else add), (g * dz).sum((0, 1))
 
@@ -39,10 +49,19 @@ KERNELS = {
     "local_write_traceable": read,
     "local_read_traceable": write,
     "local_read_add_traceable": lambda z, w, x: x + write(z, w),
-    "local_weight_grad_traceable": lambda high, low: (cells(high) * low[:, :, None]).sum((0, 1)).t().contiguous(),
+    "local_weight_grad_traceable": weight_grad,
     "lazy_workspace_update": lambda z, dz, gamma: z + gamma * dz,
     "lazy_workspace_update_backward": recur_backward,
     "lazy_workspace_update_backward_sum": lambda g, b, dz, gamma, add=None: (g + b, *recur_backward(g + b, dz, gamma, add)),
+    "all_base_b4_12_split_traceable": lambda x, a: [read(x, w) for w in a],
+    "all_base_backward": all_base_backward,
+    "final_accumulate_b4_12_traceable": lambda x, *rest: x + sum(map(write, rest[:12], rest[12:])),
+    "all_base_b4_12_grad_x": lambda g, a: sum(map(write, g, a)),
+    "all_base_b4_12_split_grad_alpha": lambda x, g: torch.stack([weight_grad(x, t) for t in g]),
+    "final_accumulate_b4_12_grad_dz_ptr": lambda g, *betas: torch.stack([read(g, b) for b in betas]),
+    "final_accumulate_b4_12_grad_beta_ptr": lambda g, *dzs: torch.stack([weight_grad(g, d) for d in dzs]),
+    "final_accumulate_list_grad_dz": lambda g, betas: [read(g, b) for b in betas],
+    "final_accumulate_list_grad_beta": lambda g, dzs: torch.stack([weight_grad(g, d) for d in dzs]),
     "gate_residual": OB.gate_residual_eager,
     "gate_residual_backward": lambda g, gate, m: ((g * m).sum(1), g * gate.unsqueeze(1)),
 }
@@ -133,6 +152,37 @@ def test_second_derivative_of_gate_residual(C):
         results.append([*first, *torch.autograd.grad(sum(g.square().sum() for g in first), leaves)])
     for a, b in zip(*results):
         torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-4)
+
+
+# ---------------------------------------------------------------------------
+# batched gradients
+# ---------------------------------------------------------------------------
+def bases(want):
+    x, alphas = leaf((2, 8, 8, 4), 0), leaf((3, 4, 16), 1)
+    return OT.all_base_b4_12_split_traceable(x, alphas), [x, alphas][want]
+
+
+def materialise(want):
+    x, dzs, betas = randn((2, 8, 8, 4), 0), [randn((2, 4, 4), 1 + i) for i in range(12)], [randn((4, 16), 13 + i) for i in range(12)]
+    leaves = [t.requires_grad_() for t in (dzs, betas)[want]]
+    return [ops.final_accumulate_b4_12_traceable(x, *dzs, *betas)], leaves
+
+
+def gate(want):
+    leaves = [leaf((2, 4, 8), 0), leaf((2, 8), 1), leaf((2, 4, 8), 2)]
+    return [OB.gate_residual(*leaves)], leaves[want]
+
+
+@pytest.mark.parametrize("node,want", [(bases, slice(0, 2)), (bases, slice(0, 1)), (materialise, 0), (materialise, 1), (gate, slice(0, 3))])
+def test_batched_gradients_are_those_of_each_sample(node, want):
+    outs, leaves = node(want)
+    grads = [randn((3, *o.shape), 40 + i) for i, o in enumerate(outs)]
+    got = torch.autograd.grad(outs, leaves, grads, is_grads_batched=True, retain_graph=True)
+    each = [torch.autograd.grad(outs, leaves, [g[i] for g in grads], retain_graph=True) for i in range(3)]
+    vmapped = torch.vmap(lambda *g: torch.autograd.grad(outs, leaves, g, retain_graph=True))(*grads)
+    for a, v, b in zip(got, vmapped, zip(*each)):
+        torch.testing.assert_close(a, torch.stack(b), rtol=1e-6, atol=1e-5)
+        torch.testing.assert_close(v, a, rtol=1e-6, atol=1e-5)
 
 
 # ---------------------------------------------------------------------------
