@@ -411,13 +411,17 @@ std::vector<Tensor> one_dtype(TensorList ts) {
   return out;
 }
 
+void check_gamma_rounded(const Tensor& alpha, TensorList betas) {
+  bool same = alpha.dim() == 2 && !betas.empty();
+  for (const Tensor& b : betas) same &= b.sizes() == alpha.sizes();
+  TORCH_CHECK_VALUE(same, "alpha [C,K] and L betas of the same shape expected, got ", shape(alpha));
+  TORCH_CHECK_VALUE(betas.size() <= LTHC_MAX_LAYERS, "depth ", betas.size(), " outside 1..", LTHC_MAX_LAYERS);
+}
+
 Tensor gamma_rounded_cuda(const Tensor& alpha_, TensorList betas_, at::ScalarType dtype) {
   on_gpu(alpha_);
   on_gpu_list(alpha_, betas_);
-  bool same = alpha_.dim() == 2 && !betas_.empty();
-  for (const Tensor& b : betas_) same &= b.sizes() == alpha_.sizes();
-  TORCH_CHECK_VALUE(same, "alpha [C,K] and L betas of the same shape expected, got ", shape(alpha_));
-  TORCH_CHECK_VALUE(betas_.size() <= LTHC_MAX_LAYERS, "depth ", betas_.size(), " outside 1..", LTHC_MAX_LAYERS);
+  check_gamma_rounded(alpha_, betas_);
   const auto betas = one_dtype(betas_);
   const Tensor alpha = alpha_.contiguous();
   const int64_t c = alpha.size(0), k = alpha.size(1);
@@ -435,6 +439,8 @@ std::tuple<Tensor, std::vector<Tensor>> gamma_rounded_backward_cuda(const Tensor
                                                                     bool need_beta) {
   on_gpu(grad_, alpha_);
   on_gpu_list(grad_, betas_);
+  check_gamma_rounded(alpha_, betas_);
+  check_like(grad_, {static_cast<int64_t>(betas_.size()), alpha_.size(0)}, "grad");
   const auto betas = one_dtype(betas_);
   const Tensor alpha = alpha_.contiguous(), grad = grad_.contiguous();
   Tensor ga = need_alpha ? at::empty_like(alpha) : at::empty({0}, alpha.options());
@@ -554,7 +560,14 @@ Tensor tri12_active_cuda(const Tensor& base, LTHC_T12(dz), const Tensor& gamma, 
 std::tuple<std::vector<Tensor>, Tensor> ws_backward_cuda(const Tensor& grad_, TensorList dzs_, const Tensor& gamma_,
                                                          int64_t L, bool want_dz) {
   on_gpu(grad_, gamma_);
+  on_gpu_list(grad_, dzs_);
   const int64_t c = grad_.size(-1), rows = c ? grad_.numel() / c : 0;
+  TORCH_CHECK_VALUE(L >= 1 && L <= kMaxWsDepth, "depth ", L, " outside 1..", kMaxWsDepth);
+  TORCH_CHECK_VALUE(gamma_.dim() == 2 && gamma_.size(0) >= L && gamma_.size(1) == c, "gamma must be [>= ", L, ", ", c,
+                    "], got ", shape(gamma_));
+  TORCH_CHECK_VALUE(dzs_.empty() || static_cast<int64_t>(dzs_.size()) >= L, "expected ", L, " dz, got ", dzs_.size());
+  for (const Tensor& dz : dzs_)
+    TORCH_CHECK_VALUE(dz.numel() == grad_.numel(), "dz ", shape(dz), " does not match grad ", shape(grad_));
   const Tensor grad = prep(grad_), gamma = gamma_.contiguous();
   std::vector<Tensor> gdz;
   if (want_dz)
@@ -562,7 +575,7 @@ std::tuple<std::vector<Tensor>, Tensor> ws_backward_cuda(const Tensor& grad_, Te
   std::vector<Tensor> dzs;
   Tensor gg = fp32_like({0}, grad), ws;
   if (!dzs_.empty()) {
-    dzs = prep_all(dzs_.slice(0, std::min<size_t>(L, dzs_.size())), grad.scalar_type());
+    dzs = prep_all(dzs_.slice(0, L), grad.scalar_type());
     gg = fp32_like({L, c}, grad);
     ws = workspace(lthc_ws_accumulate_bwd_workspace_bytes(rows, c, static_cast<int>(L)), grad);
   }
@@ -640,6 +653,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> norm_modulate_backward_cuda(const Ten
                                                                        const Tensor& inv_) {
   on_gpu(grad_, x_, weight, scale, inv_);
   const Bnc s = check_norm(x_, weight, scale, scale);
+  check_like(grad_, {s.b, s.n, s.c}, "grad");
+  TORCH_CHECK_VALUE(inv_.numel() == s.b * s.n, "inv must hold ", s.b * s.n, " values, got ", shape(inv_));
   const Tensor x = prep(x_), grad = prep_as(grad_, x.scalar_type()), w = norm_weight(weight);
   const Tensor inv = inv_.to(at::kFloat).contiguous();
   std::array<Tensor, 1> r{scale};
@@ -842,6 +857,11 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> gate_add_norm_modulat
   check_like(grad_y, {b, n, c}, "grad");
   const bool has_gd = grad_d.has_value() && grad_d->defined();
   if (has_gd) check_like(*grad_d, {b, n, c}, "grad");
+  if (has_gd) same_device(z_, *grad_d);
+  check_bnc("gate", gate, {b, c}, dt);
+  check_bnc("scale", scale, {b, c}, dt);
+  TORCH_CHECK_VALUE(has_shape(weight, {c}), "weight must be [", c, "], got ", shape(weight));
+  code(z_);
   const Tensor z = prep(z_), a = prep_as(a_, dt), gy = prep_as(grad_y, dt), w = norm_weight(weight);
   const Tensor gd = has_gd ? prep_as(*grad_d, dt) : Tensor();
   std::array<Tensor, 2> r{gate, scale};

@@ -159,3 +159,31 @@ def test_refusals():
             f()
     with pytest.raises(RuntimeError):  # functorch over an autograd node, as before
         torch.func.grad(lambda t: OB.swiglu(t).sum())(randn((2, 16), 3))
+
+
+def test_backward_operators_check_what_they_read():
+    print("case native ops: refusals of the backward operators", flush=True)
+    z, rows, row = randn((2, 3, 8), 6), randn((2, 8), 7), randn((8,), 8)
+    ganm = lambda gate=rows, scale=rows, weight=row: OB.gate_add_norm_modulate_backward(  # noqa: E731
+        None, z, z, z, gate, weight, scale, 1e-6
+    )
+    w, ggamma = randn((8, 16), 1), randn((2, 8), 9)
+    bad = [
+        (lambda: ganm(gate=rows[:1]), r"gate must be \[2, 8\]"),
+        (lambda: ganm(gate=rows.bfloat16()), "gate must be .* Float"),
+        (lambda: ganm(scale=rows[:, :4]), r"scale must be \[2, 8\]"),
+        (lambda: ganm(scale=rows.double()), "scale must be .* Float"),
+        (lambda: ganm(weight=row[:4]), r"weight must be \[8\]"),
+        (lambda: ops.norm_modulate_backward(z[:1], z, row, rows, randn((6,), 1)), r"grad must be \[2, 3, 8\]"),
+        (lambda: ops.norm_modulate_backward(z, z, row, rows, randn((5,), 1)), "inv must hold 6"),
+        (lambda: ops.lazy_gamma_rounded_backward(ggamma, w, [], True, True), "L betas"),
+        (lambda: ops.lazy_gamma_rounded_backward(ggamma, w, [w, w[:4]], True, True), "L betas"),
+        (lambda: ops.lazy_gamma_rounded_backward(ggamma[:1], w, [w, w], True, True), r"grad must be \[2, 8\]"),
+        (lambda: OT.ws_accumulate_backward(z, [z], ggamma, 2, True), "expected 2 dz, got 1"),
+        (lambda: OT.ws_accumulate_backward(z, [z, z[:1]], ggamma, 2, True), "does not match grad"),
+        (lambda: OT.ws_accumulate_backward(z, [], ggamma[:1], 2, True), r"gamma must be \[>= 2, 8\]"),
+        (lambda: OT.ws_accumulate_backward(z, [], ggamma, 25, True), "depth 25 outside"),
+    ]
+    for f, text in bad:
+        with pytest.raises(ValueError, match=text):
+            f()
