@@ -1024,6 +1024,11 @@ LTHC_OP(op_ganm_backward, "gate_add_norm_modulate_backward",
 LTHC_OP(op_gres, "gate_residual", Tensor(const Tensor&, const Tensor&, const Tensor&))
 LTHC_OP(op_gres_backward, "gate_residual_backward", std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&))
 
+#define LTHC_REPLAY(fn, name) LTHC_OP(fn, name "_backward_replay", std::vector<Tensor>(TensorList, TensorList, double))
+LTHC_REPLAY(replay_qk, "qk_norm_rope")
+LTHC_REPLAY(replay_attention, "qk_norm_rope_attention")
+LTHC_REPLAY(replay_swiglu, "swiglu")
+LTHC_REPLAY(replay_ganm, "gate_add_norm_modulate")
 LTHC_OP(op_linear_weight_grad, "linear_weight_grad", std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, bool))
 
 using BelowAutograd = at::AutoDispatchBelowADInplaceOrView;
@@ -1054,6 +1059,13 @@ struct DetachedScope {
   at::NoGradGuard no_grad;
   BelowAutograd below;
 };
+
+// Whether the call is being traced (fake, functional or other Python-dispatched tensors, as torch.compile's).  The
+// branch's nodes then differentiate the eager sequence in place of their kernels (the *_backward_replay ops): a compiled
+// graph keeps the chain's intermediates in fp32, where the kernels round at the eager ops' boundaries.
+bool traced(const Tensor& t) {
+  return t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::Functionalize}));
+}
 
 Tensor as_dtype(const Tensor& t, at::ScalarType dtype) { return t.scalar_type() == dtype ? t : t.to(dtype); }
 
@@ -1430,6 +1442,14 @@ variable_list qk_grads(AutogradContext* ctx, const Tensor& dqkv, const Tensor& d
   return {ctx->needs_input_grad(0) ? dqkv : Tensor(), row(0), row(1), Tensor(), Tensor(), Tensor()};
 }
 
+// The gradients of the first inputs that are asked for, `total` results in all.
+variable_list wanted(AutogradContext* ctx, const std::vector<Tensor>& got, size_t total) {
+  variable_list out(total);
+  for (size_t i = 0; i < got.size(); ++i)
+    if (ctx->needs_input_grad(i)) out[i] = got[i];
+  return out;
+}
+
 struct QkFn : torch::autograd::Function<QkFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& qw, const Tensor& kw,
                                const Tensor& cos, const Tensor& sin, double eps) {
@@ -1440,8 +1460,9 @@ struct QkFn : torch::autograd::Function<QkFn> {
     return {q, k};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-    DetachedScope scope;
     const auto s = ctx->get_saved_variables();
+    if (traced(s[0])) return wanted(ctx, replay_qk().call(grads, s, ctx->saved_data["eps"].toDouble()), 6);
+    DetachedScope scope;
     auto [dqkv, dw] =
         op_qk_backward().call(grads[0], grads[1], s[0], s[1], s[2], s[3], s[4], ctx->saved_data["eps"].toDouble());
     return qk_grads(ctx, dqkv, dw, s);
@@ -1457,8 +1478,9 @@ struct AttentionFn : torch::autograd::Function<AttentionFn> {
     return op_attention().call(qkv, qw, kw, cos, sin, eps);
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-    DetachedScope scope;
     const auto s = ctx->get_saved_variables();
+    if (traced(s[0])) return wanted(ctx, replay_attention().call(grads, s, ctx->saved_data["eps"].toDouble()), 6);
+    DetachedScope scope;
     auto [dqkv, dw] =
         op_attention_backward().call(grads[0], s[0], s[1], s[2], s[3], s[4], ctx->saved_data["eps"].toDouble());
     return qk_grads(ctx, dqkv, dw, s);
@@ -1472,8 +1494,10 @@ struct SwigluFn : torch::autograd::Function<SwigluFn> {
     return op_swiglu().call(x);
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const auto s = ctx->get_saved_variables();
+    if (traced(s[0])) return wanted(ctx, replay_swiglu().call(grads, s, 0.), 1);
     DetachedScope scope;
-    return {op_swiglu_backward().call(grads[0], ctx->get_saved_variables()[0])};
+    return {op_swiglu_backward().call(grads[0], s[0])};
   }
 };
 
@@ -1481,16 +1505,17 @@ struct GanmFn : torch::autograd::Function<GanmFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& z, const Tensor& a, const Tensor& gate,
                                const Tensor& weight, const Tensor& shift, const Tensor& scale, double eps) {
     BelowAutograd below;
-    ctx->save_for_backward({z, a, gate, weight, scale});
+    ctx->save_for_backward({z, a, gate, weight, shift, scale});
     ctx->saved_data["eps"] = eps;
     auto [d, y] = op_ganm().call(z, a, gate, weight, shift, scale, eps);
     return {d, y};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
-    DetachedScope scope;
     const auto s = ctx->get_saved_variables();
+    if (traced(s[0])) return wanted(ctx, replay_ganm().call(grads, s, ctx->saved_data["eps"].toDouble()), 7);
+    DetachedScope scope;
     auto [gz, ga, ggate, gw, gshift, gscale] =
-        op_ganm_backward().call(grads[0], grads[1], s[0], s[1], s[2], s[3], s[4], ctx->saved_data["eps"].toDouble());
+        op_ganm_backward().call(grads[0], grads[1], s[0], s[1], s[2], s[3], s[5], ctx->saved_data["eps"].toDouble());
     variable_list out{gz, ga, ggate, as_dtype(gw, s[3].scalar_type()), gshift, gscale, Tensor()};
     for (size_t i = 0; i < 6; ++i)
       if (!ctx->needs_input_grad(i)) out[i] = Tensor();

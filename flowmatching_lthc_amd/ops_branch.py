@@ -27,7 +27,10 @@ activation dtype), registered as a ``jit_thc`` custom op:
 Every op but block_tail (inference only) has a backward kernel of its own,
 ``jit_thc::<op>_backward``, one HIP pass that recomputes what it needs from the
 op's inputs and gives the gradients of the eager sequence.  For batched
-gradients (is_grads_batched, vmap) torch runs that pass once per sample.
+gradients (is_grads_batched, vmap) torch runs that pass once per sample.  A
+traced backward (torch.compile) differentiates the eager sequence in place of
+those kernels (gate_residual's apart, which rounds nothing in between): the
+compiled graph keeps the chain's intermediates in fp32.
 """
 
 from __future__ import annotations
@@ -70,6 +73,24 @@ def swiglu_eager(x: Tensor) -> Tensor:
 
 
 # ---------------------------------------------------------------------------
+# traced backwards: the eager sequence, differentiated
+# ---------------------------------------------------------------------------
+def _backward_replay(name: str, eager, leaves: int) -> None:
+    """Define jit_thc::<name>_backward_replay(grads, saved, eps) -> the gradients of the first `leaves` of eager's
+    arguments (saved; eps).  Composite: the native nodes call it where a backward is traced (csrc/torch_ops.cpp)."""
+
+    def replay(grads: list[Tensor], saved: list[Tensor], eps: float) -> list[Tensor]:
+        with torch.enable_grad():
+            args = [t.detach().requires_grad_(i < leaves) for i, t in enumerate(saved)]
+            outs = eager(args, eps)
+            return list(torch.autograd.grad(outs, args[:leaves], grads))
+
+    op = f"jit_thc::{name}_backward_replay"
+    torch.library.define(op, "(Tensor[] grads, Tensor[] saved, float eps) -> Tensor[]")
+    torch.library.impl(op, "CompositeImplicitAutograd")(replay)
+
+
+# ---------------------------------------------------------------------------
 # jit_thc::qk_norm_rope
 # ---------------------------------------------------------------------------
 @torch.library.custom_op("jit_thc::qk_norm_rope", mutates_args=())
@@ -96,6 +117,9 @@ def qk_norm_rope_backward(
 @_fake(qk_norm_rope_backward)
 def _(grad_q, grad_k, qkv, q_weight, k_weight, cos, sin, eps):
     return torch.empty_like(qkv), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
+
+
+_backward_replay("qk_norm_rope", lambda a, eps: list(qk_norm_rope_eager(*a, eps)), 3)
 
 
 # ---------------------------------------------------------------------------
@@ -154,6 +178,22 @@ def _(grad, qkv, q_weight, k_weight, cos, sin, eps):
     return torch.empty_like(qkv), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
 
 
+def _attention_fp32_recompute(qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos: Tensor, sin: Tensor, eps: float):
+    """qk_norm_rope_attention_eager's function with the attention itself in fp32 matrix products and softmax
+    (softmax(q k^T / sqrt(64)) v, rounded once to qkv's dtype).  Plain products, not the SDPA kernels: the ROCm
+    flash-attention backward returns gradient strides its meta function does not predict, which compiled graphs
+    assert on."""
+    q, k = qk_norm_rope_eager(qkv, q_weight, k_weight, cos, sin, eps)
+    v = qkv[:, :, 2]
+    q, k, v = (t.transpose(1, 2).float().contiguous() for t in (q, k, v))
+    kt = k.transpose(-1, -2).contiguous()
+    p = torch.softmax(torch.matmul(q, kt) * (QK_HEAD_DIM**-0.5), dim=-1)
+    return torch.matmul(p, v).to(qkv.dtype).transpose(1, 2)
+
+
+_backward_replay("qk_norm_rope_attention", lambda a, eps: [_attention_fp32_recompute(*a, eps)], 3)
+
+
 # ---------------------------------------------------------------------------
 # jit_thc::swiglu
 # ---------------------------------------------------------------------------
@@ -177,6 +217,9 @@ def swiglu_backward(grad: Tensor, x: Tensor) -> Tensor:
 @_fake(swiglu_backward)
 def _(grad, x):
     return torch.empty_like(x)
+
+
+_backward_replay("swiglu", lambda a, eps: [swiglu_eager(*a)], 1)
 
 
 # ---------------------------------------------------------------------------
@@ -227,6 +270,9 @@ def _(grad_d, grad_y, z, a, gate, weight, scale, eps):
     b, _, c = z.shape
     row = lambda: z.new_empty((b, c))  # noqa: E731
     return torch.empty_like(z), torch.empty_like(z), row(), z.new_empty((c,), dtype=_grad_dtype(weight)), row(), row()
+
+
+_backward_replay("gate_add_norm_modulate", lambda a, eps: list(gate_add_norm_modulate_eager(*a, eps)), 6)
 
 
 @torch.library.custom_op("jit_thc::gate_residual", mutates_args=())

@@ -7,6 +7,7 @@ import math
 
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from flowmatching_lthc_amd import ops
 from flowmatching_lthc_amd import ops_branch as OB
@@ -232,3 +233,47 @@ def test_gradients_of_meta_tensors(name):
     assert any(g is not None for g in grads)
     for g, a in zip(grads, leaves):
         assert g is None or (g.shape, g.dtype, g.device) == (a.shape, a.dtype, a.device)
+
+
+# ---------------------------------------------------------------------------
+# tracing
+# ---------------------------------------------------------------------------
+def trace(op, tensors, diff, **kw):
+    """The graph of op's gradients for its first `diff` operands, traced on fake tensors."""
+
+    def step(grads, *tensors):
+        leaves = [t.detach().requires_grad_(i < diff) for i, t in enumerate(tensors)]
+        outs = op(*leaves, **kw)
+        return torch.autograd.grad(outs, leaves[:diff], grads)
+
+    outs = op(*(t.to("meta") for t in tensors), **kw)
+    grads = [torch.zeros(o.shape, dtype=o.dtype) for o in (outs if isinstance(outs, tuple) else (outs,))]
+    graph = make_fx(step, tracing_mode="fake")(grads, *tensors).graph
+    (out,) = [n for n in graph.nodes if n.op == "output"]
+    for got, want in zip(out.args[0], tensors):
+        assert got.meta["val"].shape == want.shape and got.meta["val"].dtype == want.dtype
+    return [n for n in graph.nodes if n.op == "call_function"]
+
+
+def traced_cases():
+    z, rows, qkv, w = randn((2, 64, 8), 0).bfloat16(), randn((2, 8), 1).bfloat16(), randn((2, 64, 3, 2, 64), 2).bfloat16(), randn((64,), 3)
+    table = randn((64, 64), 4)
+    return {
+        "qk_norm_rope": (OB.qk_norm_rope, (qkv, w, w, table, table), 3, {"eps": 1e-6}),
+        "qk_norm_rope_attention": (OB.qk_norm_rope_attention, (qkv, w, w, table, table), 3, {"eps": 1e-6}),
+        "swiglu": (OB.swiglu, (randn((4, 32), 5).bfloat16(),), 1, {}),
+        "gate_add_norm_modulate": (OB.gate_add_norm_modulate, (z, z, rows, randn((8,), 6), rows, rows), 6, {"eps": 1e-6}),
+    }
+
+
+@pytest.mark.parametrize("name", traced_cases())
+def test_traced_branch_backward_is_the_eager_sequence(name):
+    """A traced graph holds the plain sequence's gradients, whose intermediates the compiler keeps in fp32, and not the
+    backward kernel, which rounds them where eager does.  The attention's products are fp32 ones (scores and output again, and four gradients)."""
+    op, tensors, diff, kw = traced_cases()[name]
+    nodes = trace(op, tensors, diff, **kw)
+    names = {str(n.target) for n in nodes}
+    assert f"jit_thc.{name}_backward.default" not in names and {n for n in names if "jit_thc" in n} <= {f"jit_thc.{name}.default"}
+    products = [n for n in nodes if n.target in (torch.ops.aten.bmm.default, torch.ops.aten.mm.default)]
+    assert len(products) == (6 if name == "qk_norm_rope_attention" else 0)
+    assert all(n.meta["val"].dtype == torch.float32 for n in products)
