@@ -9,6 +9,7 @@
 // fp32 interface training step at B = 5 0.96-1.1 -> 0.41 ms.
 
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -1698,7 +1699,14 @@ std::tuple<Tensor, Tensor> read_with_residual(const Tensor& x, const Tensor& wei
 }
 
 Tensor linear(const Tensor& x, const Tensor& weight, const std::optional<Tensor>& bias) {
-  return LinearFn::apply(x, weight, bias);
+  if (!at::autocast::is_autocast_enabled(at::kCUDA)) return LinearFn::apply(x, weight, bias);
+  // autocast's own conversion, which keeps a parameter's copy for the later calls of the region
+  const auto cast = [dt = at::autocast::get_autocast_dtype(at::kCUDA)](const Tensor& t) {
+    return at::autocast::cached_cast(dt, t, at::kCUDA);
+  };
+  std::optional<Tensor> b = bias;
+  if (b.has_value() && b->defined()) b = cast(*b);
+  return LinearFn::apply(cast(x), cast(weight), b);
 }
 
 std::vector<Tensor> lazy_workspace_step(const Tensor& z, const Tensor& dz, const Tensor& gamma, bool split) {

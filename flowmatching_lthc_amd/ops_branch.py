@@ -347,7 +347,7 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor | None:
         return None
     if dt not in (torch.bfloat16, torch.float16) or weight.device != x.device:
         return None
-    return torch.ops.jit_thc.linear(*(t.to(dt) for t in operands), *(() if bias is not None else (None,)))
+    return torch.ops.jit_thc.linear(x, weight, bias)
 
 
 # ---------------------------------------------------------------------------

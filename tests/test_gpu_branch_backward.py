@@ -235,6 +235,10 @@ def test_linear_layer_routes():
         (gw,) = torch.autograd.grad(y, layer.weight, g.bfloat16(), create_graph=True)
         second.append(torch.autograd.grad(gw.float().square().sum(), xl)[0])
     assert rel(*second) <= 1e-2
+    amp = M.CastLinear(64, 136).to(DEV)
+    with torch.autocast("cuda", dtype=torch.bfloat16):  # a parameter is converted once in an autocast region
+        nodes = [amp(x).grad_fn for _ in range(2)]
+    assert [f for f, _ in nodes[0].next_functions[1:]] == [f for f, _ in nodes[1].next_functions[1:]]
     lin.weight.requires_grad_(False)
     assert OB.linear(xl, lin.weight, lin.bias) is None and lin(xl).requires_grad
     lin.weight.requires_grad_(True)
