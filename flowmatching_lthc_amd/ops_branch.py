@@ -38,6 +38,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 from torch import Tensor
+from torch.utils._device import DeviceContext
 
 from . import _abi
 from .ops import _fake, _refuse
@@ -300,8 +301,11 @@ def _(grad, gate, m):
 # ---------------------------------------------------------------------------
 # linear layers in training: weight and bias gradients in one pass over the rows
 # ---------------------------------------------------------------------------
-# Below this many rows torch's product and column sum take as long (M = 512, N = 4096, K = 768, bf16: 29 us against 30;
-# M = 8192: 106 us against 89).
+# From here the kernel is as fast as torch's product and column sum, or faster, on every layer shape of the models (N x K,
+# bf16, us of the kernel / torch's).  512 rows: 4096 x 768 28.5 / 27.1 (the one shape behind, with 768 rows too: 29.1 /
+# 27.7), 2304 x 768 21.9 / 28.4, 768 x 2048 20.5 / 26.8, 768 x 768 16.5 / 26.6, 6144 x 1152 30.9 / 34.0, 192 x 192
+# 13.2 / 37.2, 128 x 48 12.2 / 18.8.  1024 rows: 30.2 / 31.0, 26.4 / 28.4, 25.2 / 27.0, 19.7 / 26.7.  256 rows: 21.9 /
+# 25.0, 18.2 / 23.8, 16.9 / 23.8, 14.9 / 23.7, so the line could lie lower.
 LINEAR_MIN_ROWS = 512
 
 
@@ -321,11 +325,14 @@ def _(grad, x, need_bias):
 def linear(x: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor | None:
     """F.linear(x, weight, bias) with the weight and bias gradients of a training step from linear_weight_grad, or None
     where that does not apply and the caller calls F.linear: no gradient of the weight, not 16-bit products (autocast's,
-    or the operands' own), few rows, or tracing, functorch and forward-mode transforms, which know torch's linear."""
+    or the operands' own), few rows, or tracing, functorch and forward-mode transforms, tensor subclasses and torch
+    function and dispatch modes (a flop counter, for one), which know torch's linear."""
     if torch.compiler.is_compiling() or not (
         torch.is_grad_enabled()
         and weight.requires_grad
         and type(x) is Tensor
+        and type(weight) in (Tensor, torch.nn.Parameter)
+        and type(bias) in (Tensor, torch.nn.Parameter, type(None))
         and x.is_cuda
         and x.dim() >= 2
         and x.is_floating_point()
@@ -335,6 +342,8 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor | None:
         and x.shape[-1] == weight.shape[1]
         and torch._C._functorch.peek_interpreter_stack() is None
         and torch.autograd.forward_ad._current_level < 0
+        and torch._C._len_torch_dispatch_stack() == 0
+        and all(type(m) is DeviceContext for m in map(torch._C._get_function_stack_at, range(torch._C._len_torch_function_stack())))
     ):
         return None
     dt = x.dtype

@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import pytest
 import torch
+from torch.utils.flop_counter import FlopCounterMode
 
 from flowmatching_lthc_amd import model as M
 from flowmatching_lthc_amd import ops
@@ -248,3 +249,42 @@ def test_linear_layer_routes():
     assert rel(torch.func.grad(lambda t: lin(t).float().sum())(x.bfloat16()), out) <= 1e-6
     with torch.no_grad():
         assert OB.linear(xl, lin.weight, None) is None
+
+
+class SeenLinear(torch.nn.Parameter):
+    """A parameter that notes the calls of torch's linear that it takes part in."""
+
+    seen = 0
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen += func is torch.nn.functional.linear
+        with torch._C.DisableTorchFunctionSubclass():
+            return func(*args, **(kwargs or {}))
+
+
+class Seen(torch.overrides.TorchFunctionMode):
+    seen = 0
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen += func is torch.nn.functional.linear
+        return func(*args, **(kwargs or {}))
+
+
+def test_linear_layer_is_torchs_own_to_subclasses_and_modes():
+    """What takes torch's linear apart sees it: a parameter subclass, a torch function mode, a flop counter (three
+    products of 2 M N K).  A default device is no such mode."""
+    print("case linear layer: subclasses and modes", flush=True)
+    lin, x = M.CastLinear(64, 128).to(DEV).bfloat16(), torch.ones((600, 64), device=DEV, dtype=torch.bfloat16)
+    x.requires_grad_()
+    with FlopCounterMode(display=False) as flops:
+        lin(x).sum().backward()
+    assert flops.get_total_flops() == 3 * 2 * 600 * 64 * 128
+    with Seen() as mode:
+        lin(x)
+    assert mode.seen == 1
+    with torch.device(DEV):
+        assert OB.linear(x, lin.weight, lin.bias) is not None
+    lin._parameters["weight"] = torch.Tensor._make_subclass(SeenLinear, lin.weight.detach(), True)
+    lin(x)
+    assert SeenLinear.seen == 1
