@@ -117,7 +117,7 @@ def qk_norm_rope_backward(
 
 @_fake(qk_norm_rope_backward)
 def _(grad_q, grad_k, qkv, q_weight, k_weight, cos, sin, eps):
-    return torch.empty_like(qkv), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
+    return qkv.new_empty(qkv.shape), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
 
 
 _backward_replay("qk_norm_rope", lambda a, eps: list(qk_norm_rope_eager(*a, eps)), 3)
@@ -176,7 +176,7 @@ def qk_norm_rope_attention_backward(
 
 @_fake(qk_norm_rope_attention_backward)
 def _(grad, qkv, q_weight, k_weight, cos, sin, eps):
-    return torch.empty_like(qkv), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
+    return qkv.new_empty(qkv.shape), qkv.new_empty((2, QK_HEAD_DIM), dtype=torch.float32)
 
 
 def _attention_fp32_recompute(qkv: Tensor, q_weight: Tensor, k_weight: Tensor, cos: Tensor, sin: Tensor, eps: float):
@@ -217,7 +217,7 @@ def swiglu_backward(grad: Tensor, x: Tensor) -> Tensor:
 
 @_fake(swiglu_backward)
 def _(grad, x):
-    return torch.empty_like(x)
+    return x.new_empty(x.shape)
 
 
 _backward_replay("swiglu", lambda a, eps: [swiglu_eager(*a)], 1)
@@ -270,7 +270,7 @@ def gate_add_norm_modulate_backward(
 def _(grad_d, grad_y, z, a, gate, weight, scale, eps):
     b, _, c = z.shape
     row = lambda: z.new_empty((b, c))  # noqa: E731
-    return torch.empty_like(z), torch.empty_like(z), row(), z.new_empty((c,), dtype=_grad_dtype(weight)), row(), row()
+    return z.new_empty(z.shape), z.new_empty(z.shape), row(), z.new_empty((c,), dtype=_grad_dtype(weight)), row(), row()
 
 
 _backward_replay("gate_add_norm_modulate", lambda a, eps: list(gate_add_norm_modulate_eager(*a, eps)), 6)
@@ -295,7 +295,7 @@ def gate_residual_backward(grad: Tensor, gate: Tensor, m: Tensor) -> tuple[Tenso
 
 @_fake(gate_residual_backward)
 def _(grad, gate, m):
-    return grad.new_empty(gate.shape), torch.empty_like(m)
+    return grad.new_empty(gate.shape), m.new_empty(m.shape)
 
 
 # ---------------------------------------------------------------------------

@@ -488,7 +488,7 @@ def all_base_backward(
 
 @_fake(all_base_backward)
 def _(x0: Tensor, grads: list[Tensor], alpha_stack: Tensor, need_x: bool, need_alpha: bool):
-    gx = torch.empty_like(x0) if need_x else x0.new_empty((0,))
+    gx = x0.new_empty(x0.shape if need_x else (0,))
     return gx, x0.new_empty((len(grads), x0.shape[3], K) if need_alpha else (0,), dtype=torch.float32)
 
 

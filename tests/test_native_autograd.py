@@ -277,3 +277,20 @@ def test_traced_branch_backward_is_the_eager_sequence(name):
     products = [n for n in nodes if n.target in (torch.ops.aten.bmm.default, torch.ops.aten.mm.default)]
     assert len(products) == (6 if name == "qk_norm_rope_attention" else 0)
     assert all(n.meta["val"].dtype == torch.float32 for n in products)
+
+
+def test_fake_gradients_are_contiguous():
+    """The backward kernels return contiguous gradients whatever the strides of their operands; so do their fakes, whose
+    strides a compiled graph asserts."""
+    z, rows, w = meta(4, 2, 8).transpose(0, 1), meta(2, 8), meta(8)
+    x0, qkv = meta(2, 8, 8, 8).permute(0, 2, 1, 3), meta(4, 2, 3, 2, 64).transpose(0, 1)
+    q, n, table = meta(2, 4, 2, 64), meta(64), meta(4, 64)
+    outs = [
+        *OB.qk_norm_rope_backward(q, q, qkv, n, n, table, table, 1e-6),
+        *OB.qk_norm_rope_attention_backward(q, qkv, n, n, table, table, 1e-6),
+        OB.swiglu_backward(meta(2, 4, 4), z),
+        *OB.gate_add_norm_modulate_backward(None, z, z, z, rows, w, rows, 1e-6),
+        *OB.gate_residual_backward(z, rows, z),
+        *OT.all_base_backward(x0, [z], meta(1, 8, 16), True, True),
+    ]
+    assert all(o.is_contiguous() for o in outs)
