@@ -255,9 +255,5 @@ def recur_bwd_workspace_bytes(rows: int, C: int) -> int:
     return int(load().lthc_recur_bwd_workspace_bytes(rows, C))
 
 
-def norm_modulate_bwd_workspace_bytes(B: int, N: int, C: int) -> int:
-    return int(load().lthc_norm_modulate_bwd_workspace_bytes(B, N, C))
-
-
 def ws_accumulate_bwd_workspace_bytes(rows: int, C: int, L: int) -> int:
     return int(load().lthc_ws_accumulate_bwd_workspace_bytes(rows, C, L))
