@@ -307,6 +307,11 @@ def _(grad, gate, m):
 # 13.2 / 37.2, 128 x 48 12.2 / 18.8.  1024 rows: 30.2 / 31.0, 26.4 / 28.4, 25.2 / 27.0, 19.7 / 26.7.  256 rows: 21.9 /
 # 25.0, 18.2 / 23.8, 16.9 / 23.8, 14.9 / 23.7, so the line could lie lower.
 LINEAR_MIN_ROWS = 512
+# From one 256 x 128 tile of the weight per CU on, torch's tiles are the better ones (rounds of whole tiles; us of the
+# kernel / torch's at 512, 4096 and 16384 rows).  216 tiles, 6144 x 1152: 30.9 / 34.0, 82.6 / 93.4, 261 / 289; 256, 4096 x
+# 2048: 29.8 / 28.6, 85.0 / 87.4, 272 / 285; 344, 2048 x 5456: 39.2 / 40.2, 133 / 115, 460 / 363; 384, 6144 x 2048: 40.9 /
+# 33.1, 135 / 113, 469 / 383; 512, 4096 x 4096: 46.7 / 35.9, 154 / 136, 537 / 482.
+LINEAR_MAX_TILES = 256
 
 
 @torch.library.custom_op("jit_thc::linear_weight_grad", mutates_args=())
@@ -325,7 +330,7 @@ def _(grad, x, need_bias):
 def linear(x: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor | None:
     """F.linear(x, weight, bias) with the weight and bias gradients of a training step from linear_weight_grad, or None
     where that does not apply and the caller calls F.linear: no gradient of the weight, not 16-bit products (autocast's,
-    or the operands' own), few rows, or tracing, functorch and forward-mode transforms, tensor subclasses and torch
+    or the operands' own), few rows, a wide weight, or tracing, functorch and forward-mode transforms, tensor subclasses and torch
     function and dispatch modes (a flop counter, for one), which know torch's linear."""
     if torch.compiler.is_compiling() or not (
         torch.is_grad_enabled()
@@ -340,6 +345,7 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor | None:
         and x.shape[-1] % 8 == 0
         and weight.shape[0] % 8 == 0
         and x.shape[-1] == weight.shape[1]
+        and -(-weight.shape[0] // 256) * -(-weight.shape[1] // 128) < LINEAR_MAX_TILES
         and torch._C._functorch.peek_interpreter_stack() is None
         and torch.autograd.forward_ad._current_level < 0
         and torch._C._len_torch_dispatch_stack() == 0

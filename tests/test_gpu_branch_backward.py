@@ -184,9 +184,12 @@ def test_qk_norm_rope_backward(B, N, H, dtype, tdt, wdt):
     assert ours[0][:, :, 2].abs().max().item() == 0.0
 
 
-# ends of the 256 x 128 tile and of the 32-row stage, one stage, an odd number of stages, parts that end inside a stage,
-# fewer tiles and more tiles than blocks fit at once
-@pytest.mark.parametrize("rows,N,K", [(1, 8, 8), (33, 264, 136), (96, 256, 128), (1000, 48, 768), (4097, 520, 392), (600, 4096, 2048)])
+# ends of the 256 x 128 tile and of the 32-row stage, one stage, an odd number of stages, parts that end inside a stage;
+# one tile per CU, parts long enough for two blocks per CU (16417 rows in 9 parts), more tiles than fit at once (561)
+@pytest.mark.parametrize("rows,N,K", [
+    (1, 8, 8), (33, 264, 136), (96, 256, 128), (1000, 48, 768), (4097, 520, 392), (600, 4096, 2048),
+    (16384 + 33, 2304, 768), (300, 8200, 2056),
+])  # fmt: skip
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_linear_weight_grad(rows, N, K, dtype):
     print(f"case linear weight grad rows={rows} N={N} K={K} {dtype}", flush=True)
@@ -243,6 +246,9 @@ def test_linear_layer_routes():
     lin.weight.requires_grad_(False)
     assert OB.linear(xl, lin.weight, lin.bias) is None and lin(xl).requires_grad
     lin.weight.requires_grad_(True)
+    wide = torch.zeros((4096, 2048), device=DEV, dtype=torch.bfloat16, requires_grad=True)  # 256 tiles, and 240
+    rows = torch.zeros((512, 2048), device=DEV, dtype=torch.bfloat16)
+    assert OB.linear(rows, wide, None) is None and OB.linear(rows, wide[:3840], None) is not None
     w = lin.weight.detach()
     assert OB.linear(xl[:1, :100], lin.weight, None) is None and OB.linear(x, lin.weight, None) is None
     out = torch.func.grad(lambda t: torch.nn.functional.linear(t, w).float().sum())(x.bfloat16())
