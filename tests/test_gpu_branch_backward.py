@@ -92,8 +92,10 @@ def norm_mod_exact(x, w, shift, scale):
 
 
 # C: below and past one 256-channel chunk, the 3-chunk form and the widest; N: one token, runs that end inside a block,
-# a sample longer than a block's run; B * N large enough for the 16-token runs (1, 8192) and larger (40, 1030)
-@pytest.mark.parametrize("B,N,C", [(2, 1, 8), (3, 9, 260), (2, 257, 768), (1, 8192, 64), (40, 1030, 128), (2, 33, 1152), (2, 5, 2048)])
+# a sample longer than a block's run; B * N large enough for the 16-token runs (1, 8192) and larger (40, 1030); column
+# sums of many parts over few columns (1, 8192) and from 12288 columns on (16, 272, 768); one block per CU (8, 520, 1280)
+@pytest.mark.parametrize("B,N,C", [(2, 1, 8), (3, 9, 260), (2, 257, 768), (1, 8192, 64), (40, 1030, 128), (2, 33, 1152),
+                                   (2, 5, 2048), (16, 272, 768), (8, 520, 1280)])  # fmt: skip
 @pytest.mark.parametrize("dtype,wdt", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
 def test_gated_norm_backward(B, N, C, dtype, wdt):
     print(f"case gated norm backward B={B} N={N} C={C} {dtype} {wdt}", flush=True)
