@@ -6,7 +6,8 @@ views of the projection; chunk + F.silu + mul), so the check covers the exact op
 for.  fp32: max|d| / max|ref| <= 1e-6.  16-bit: the kernels reproduce every eager rounding, so at least
 99 % of the elements are bit-identical and none differs by more than one unit in the last place
 (|d| <= 2^-7 |ref| for bf16, 2^-10 |ref| for fp16) -- a reduction-order difference in the fp32 mean can
-move one rounding.  Gradients (recomputed through the eager sequence) equal the eager model's.
+move one rounding.  Gradients, from backward kernels that keep the eager roundings or sum in fp32 where eager rounds,
+agree with the eager model's.
 """
 
 from __future__ import annotations
@@ -269,9 +270,8 @@ def test_qk_norm_rope_attention_table_and_weight_formats(dtype, N):
 
 
 def test_qk_norm_rope_attention_gradients_and_errors():
-    """The backward (recomputed through the eager q/k norm + RoPE sequence, the attention itself in fp32 products)
-    matches autograd of the eager sequence to 1e-2 of each gradient's scale; unsupported shapes and dtypes raise
-    ValueError."""
+    """The backward (one kernel; 16-bit matrix operands, fp32 sums) matches autograd of the eager sequence to 1e-2 of each
+    gradient's scale; unsupported shapes and dtypes raise ValueError."""
     print("case attention gradients", flush=True)
     B, N, H = 2, 256, 4
     gen = torch.Generator().manual_seed(8)
