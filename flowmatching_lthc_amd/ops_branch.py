@@ -332,7 +332,7 @@ def linear(x: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor | None:
     where that does not apply and the caller calls F.linear: no gradient of the weight, not 16-bit products (autocast's,
     or the operands' own), few rows, a wide weight, or tracing, functorch and forward-mode transforms, tensor subclasses and torch
     function and dispatch modes (a flop counter, for one), which know torch's linear."""
-    if torch.compiler.is_compiling() or not (
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or not (
         torch.is_grad_enabled()
         and weight.requires_grad
         and type(x) is Tensor

@@ -281,7 +281,7 @@ class Seen(torch.overrides.TorchFunctionMode):
 
 def test_linear_layer_is_torchs_own_to_subclasses_and_modes():
     """What takes torch's linear apart sees it: a parameter subclass, a torch function mode, a flop counter (three
-    products of 2 M N K).  A default device is no such mode."""
+    products of 2 M N K), the TorchScript tracer.  A default device is no such mode."""
     print("case linear layer: subclasses and modes", flush=True)
     lin, x = M.CastLinear(64, 128).to(DEV).bfloat16(), torch.ones((600, 64), device=DEV, dtype=torch.bfloat16)
     x.requires_grad_()
@@ -293,6 +293,7 @@ def test_linear_layer_is_torchs_own_to_subclasses_and_modes():
     assert mode.seen == 1
     with torch.device(DEV):
         assert OB.linear(x, lin.weight, lin.bias) is not None
+    assert "aten::linear" in str(torch.jit.trace(lin, x).graph)
     lin._parameters["weight"] = torch.Tensor._make_subclass(SeenLinear, lin.weight.detach(), True)
     lin(x)
     assert SeenLinear.seen == 1
